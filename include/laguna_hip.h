@@ -288,6 +288,13 @@ int lq_q8_prefill_attn(const uint16_t* q, const uint8_t* kc, const uint16_t* ks,
                        int64_t Hq, int64_t Hkv, int64_t L, int64_t D, int64_t cap, int64_t n,
                        float scale, uint16_t* out, void* stream);
 
+/* lq_q8_prefill_attn for any grouping of up to 64 query heads per KV head. */
+int lq_q8_prefill_attn_grouped(const uint16_t* q, const uint8_t* kc, const uint16_t* ks,
+                               const uint16_t* kb, const uint8_t* vc, const uint16_t* vs,
+                               const uint16_t* vb, int64_t B, int64_t Hq, int64_t Hkv, int64_t L,
+                               int64_t D, int64_t cap, int64_t n, float scale, uint16_t* out,
+                               void* stream);
+
 /*
  * The input half of a decode step's attention block in one launch (one input row; laguna.py's
  * input_layernorm, then laguna.py:97-101 at L = 1): y = W (RMSNorm(x) * norm_w) as lq_gemv_fused

@@ -54,6 +54,8 @@ SIGNATURES = {
                                             vp, i64, vp]),
     "lq_q8_prefill_attn": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64,
                                  f32, vp, vp]),
+    "lq_q8_prefill_attn_grouped": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64,
+                                         i64, f32, vp, vp]),
     "lq_gemv_norm_rope": (i32, [vp, vp, vp, vp, i64, i64, f32, vp, vp, i64, i64, f32, vp, i64, f32,
                                 i64, vp, vp, vp]),
     "lq_q8_decode_append_attn_pos": (i32, [vp, vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64,

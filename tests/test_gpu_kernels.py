@@ -883,3 +883,22 @@ def test_prefill_never_materializes_scores(dev):
     qs = q[:, :, 2040:].float().cpu().numpy()
     want = A.fused_attention(qs, kn, vn, 10240, 0.09, causal=True)
     assert_attn_close(out[:, :, 2040:], want, "prefill rows 2040..2047 at 10,240")
+
+
+@pytest.mark.parametrize("n,L,G,Hkv,B", [(300, 17, 3, 2, 1), (257, 43, 6, 1, 1), (128, 128, 6, 2, 1),
+                                         (1000, 52, 5, 2, 2), (700, 17, 64, 1, 1),
+                                         (2100, 130, 12, 1, 1), (129, 86, 3, 3, 1)])
+def test_prefill_of_any_grouping_matches_the_blocked_path(dev, n, L, G, Hkv, B):
+    """Groupings that are no power of two (a 256-row block then ends inside a position, 258 = 43 x 6
+    rows leave two for the next block) and up to 64: the prefill kernel against the verify kernel's
+    blocks and the float64 oracle, at the attention tolerance."""
+    from lagunalab_amd.q8_attn import _prefill_blocked, q8_prefill_attention
+    rng = np.random.default_rng(n + L + G)
+    kq, vq = make_cache(rng, B, Hkv, n, n + 5, dev)
+    q = Q.randn_bf16(rng, (B, Hkv * G, L, 128))
+    qd = to_dev_bf16(q, dev)
+    got = q8_prefill_attention(qd, kq, vq, n, 0.09)
+    assert_attn_close(got, _prefill_blocked(qd, kq, vq, n, 0.09).float().cpu().numpy(),
+                      "against the blocked path")
+    assert_attn_close(got, A.fused_attention(q, cache_np(kq), cache_np(vq), n, 0.09, causal=True),
+                      "against the oracle")

@@ -110,3 +110,71 @@ def test_v_scales_changing_across_the_cache(dev, B):
         assert mag < 2.0 ** -14, mag  # the output is the small-scale region's
         assert_attn_close(got[sl], want, f"V scales jumping by 2^10 and 2^20, sequence {b}",
                           2e-3 * mag, RTOL)
+
+
+# ------------------------------------------------------------------------------------- prefill
+# For groupings other than 1, 2, 4 and 8 the prefill kernel takes q, K and V in fp16 with
+# power-of-two factors per tile; the float64 oracle bounds it by the operands' 2^-11 steps: a score of size s moves by about s 2^-11 (peaked
+# scores are why the wide-q cases use fewer, smaller keys), P and V by 2^-11 relative each.
+
+@pytest.mark.parametrize("G", [6, 3])
+@pytest.mark.parametrize("qstd,kstd,vstd", [(1e-4, 1.0, 1.0), (1.0, 1.0, 1e-6), (1.0, 1.0, 1e5),
+                                            (2e5, 1e-5, 1.0), (1e-4, 3e5, 1.0), (2e5, 1e-5, 1e6),
+                                            (3.0, 1e-3, 1e-4)])
+def test_prefill_operand_range(dev, G, qstd, kstd, vstd):
+    """A 37-row chunk behind 963 rows: q, K and V far outside fp16's range on either side."""
+    from lagunalab_amd.q8_attn import q8_prefill_attention
+    rng = np.random.default_rng(int(qstd * 3 + vstd * 5) % 1000 + G)
+    n, L, Hkv, cap = 1000, 37, 2, 1024
+    caches = []
+    for std in (kstd, vstd):
+        x = Q.round_bf16(Q.randn_bf16(rng, (1, Hkv, n, 128)) * np.float32(std))
+        from lagunalab_amd.quant import quantize_into
+        c = (torch.zeros((1, Hkv, cap, 128), dtype=torch.uint8, device=dev),
+             torch.zeros((1, Hkv, cap, 2), dtype=torch.bfloat16, device=dev),
+             torch.zeros((1, Hkv, cap, 2), dtype=torch.bfloat16, device=dev))
+        quantize_into(to_dev_bf16(x, dev), *c, 0, 64, 8)
+        caches.append(c)
+    q = Q.round_bf16(Q.randn_bf16(rng, (1, Hkv * G, L, 128)) * np.float32(qstd))
+    got = q8_prefill_attention(to_dev_bf16(q, dev), *caches, n, 128 ** -0.5)
+    assert torch.isfinite(got.float()).all()
+    want = A.fused_attention(q, cache_np(caches[0]), cache_np(caches[1]), n, 128 ** -0.5,
+                             causal=True)
+    s = max(1.0, qstd * kstd)  # largest scores ~5 s nats, each off by up to 2^-11 of its terms
+    assert_attn_close(got, want, f"prefill G={G} q {qstd} K {kstd} V {vstd}", 2e-3 * s * vstd, RTOL)
+
+
+@pytest.mark.parametrize("G", [6, 3])
+def test_prefill_factors_change_between_tiles(dev, G):
+    """K and V whose sizes jump by powers of two between 300-row regions (so that tiles straddle
+    them): the V factor rises and falls, K's factor moves q's. The keys of the smallest-V region
+    get the largest scores. (V sizes 2^-20 apart at most: where a tile straddles the regions, the
+    small values stay normal fp16 numbers below a largest one of 2^12 to 2^15.)"""
+    from lagunalab_amd.q8_attn import q8_prefill_attention
+    from lagunalab_amd.quant import quantize_into
+    rng = np.random.default_rng(78)
+    n, cap, Hkv, L = 3000, 3072, 2, 70
+    region = (np.arange(n) // 300) % 3
+    q = Q.randn_bf16(rng, (1, Hkv, 1, 1, 128)) * np.float32(4.0)
+    q = Q.round_bf16(q + 0.3 * Q.randn_bf16(rng, (1, Hkv, G, L, 128))).reshape(1, Hkv * G, L, 128)
+    qdir = q[0, ::G, 0] / np.linalg.norm(q[0, ::G, 0], axis=-1, keepdims=True)
+    shift = np.where(region == 1, 6.0, -6.0).astype(np.float32)
+    k = Q.randn_bf16(rng, (1, Hkv, n, 128)) + shift[None, None, :, None] * qdir[None, :, None, :]
+    k[:, :, region == 2] *= np.float32(2.0 ** -12)
+    v = Q.randn_bf16(rng, (1, Hkv, n, 128)) * (np.float32(2.0) ** np.array([5, -15, -5])[region]
+                                               ).astype(np.float32)[None, None, :, None]
+    caches = []
+    for x in (k, v):
+        c = (torch.zeros((1, Hkv, cap, 128), dtype=torch.uint8, device=dev),
+             torch.zeros((1, Hkv, cap, 2), dtype=torch.bfloat16, device=dev),
+             torch.zeros((1, Hkv, cap, 2), dtype=torch.bfloat16, device=dev))
+        quantize_into(to_dev_bf16(Q.round_bf16(x), dev), *c, 0, 64, 8)
+        caches.append(c)
+    got = q8_prefill_attention(to_dev_bf16(q, dev), *caches, n, 128 ** -0.5)
+    want = A.fused_attention(q, cache_np(caches[0]), cache_np(caches[1]), n, 128 ** -0.5,
+                             causal=True)
+    assert torch.isfinite(got.float()).all()
+    # each row against its own largest value: the rows rest on different regions
+    mag = np.abs(want).max(-1, keepdims=True)
+    err = np.abs(got.float().cpu().numpy() - want)
+    assert np.all(err <= 8e-3 * mag + RTOL * np.abs(want)), float((err / mag).max())
