@@ -288,12 +288,18 @@ int lq_q8_prefill_attn(const uint16_t* q, const uint8_t* kc, const uint16_t* ks,
                        int64_t Hq, int64_t Hkv, int64_t L, int64_t D, int64_t cap, int64_t n,
                        float scale, uint16_t* out, void* stream);
 
-/* lq_q8_prefill_attn for any grouping of up to 64 query heads per KV head. */
+/*
+ * lq_q8_prefill_attn for any grouping of up to 64 query heads per KV head. Chunks whose blocks of
+ * 256 rows would leave CUs idle have their keys split over workgroups; the partial rows need
+ * lq_prefill_workspace_bytes of scratch (0 for chunks that are not split; negative on bad
+ * arguments; at most about 70 MB), of any contents and free again when the call's work is done.
+ */
+int64_t lq_prefill_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t n);
 int lq_q8_prefill_attn_grouped(const uint16_t* q, const uint8_t* kc, const uint16_t* ks,
                                const uint16_t* kb, const uint8_t* vc, const uint16_t* vs,
                                const uint16_t* vb, int64_t B, int64_t Hq, int64_t Hkv, int64_t L,
                                int64_t D, int64_t cap, int64_t n, float scale, uint16_t* out,
-                               void* stream);
+                               void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
  * The input half of a decode step's attention block in one launch (one input row; laguna.py's

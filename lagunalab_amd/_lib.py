@@ -54,8 +54,9 @@ SIGNATURES = {
                                             vp, i64, vp]),
     "lq_q8_prefill_attn": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64,
                                  f32, vp, vp]),
+    "lq_prefill_workspace_bytes": (i64, [i64, i64, i64, i64, i64]),
     "lq_q8_prefill_attn_grouped": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64,
-                                         i64, f32, vp, vp]),
+                                         i64, f32, vp, vp, i64, vp]),
     "lq_gemv_norm_rope": (i32, [vp, vp, vp, vp, i64, i64, f32, vp, vp, i64, i64, f32, vp, i64, f32,
                                 i64, vp, vp, vp]),
     "lq_q8_decode_append_attn_pos": (i32, [vp, vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64,

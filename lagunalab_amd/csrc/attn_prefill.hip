@@ -125,38 +125,70 @@ struct PrefillSmem {
   alignas(16) _Float16 vt[D * PT];  // [dim][slot], 16-byte chunk j of dim d at chunk j ^ (d & 15)
 };
 
-template <bool RANGE>
+struct PrefillSplit {
+  FastDiv g;        // division by G
+  int shares;       // workgroups per KV head
+  int tiles;        // tiles of a share; 0: every workgroup takes one whole block
+  float* part_o;    // [2 x workgroups][PROWS][D] partial rows of shares (slot 2 x + 1: the part
+  float2* part_ml;  // begins its block), normalized, and their (max in log2 units, sum)
+};
+
+// Key tiles of position block pb.
+__host__ __device__ __forceinline__ int prefill_tiles(int pb, int R, FastDiv g, int base) {
+  return (base + (int)fdiv_u((uint32_t)min(pb * PROWS + PROWS - 1, R - 1), g)) / PT + 1;
+}
+
+template <bool RANGE, bool SPLIT>
 __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
     const uint16_t* __restrict__ q, const uint8_t* __restrict__ kc,
     const uint16_t* __restrict__ ks, const uint16_t* __restrict__ kb,
     const uint8_t* __restrict__ vc, const uint16_t* __restrict__ vs,
     const uint16_t* __restrict__ vb, uint16_t* __restrict__ out, int64_t cap, int n, int L,
-    int Hkv, int G, int npb, float q_scale, float k_scale) {
+    int Hkv, int G, int npb, PrefillSplit sp, float q_scale, float k_scale) {
   __shared__ PrefillSmem sm;
-  const int tid = threadIdx.x;
+  const int x = blockIdx.x;
+  const int hk = x % Hkv;  // consecutive workgroups (consecutive XCDs) take consecutive KV heads
+  const int share = (x / Hkv) % sp.shares;
+  const int b = x / (Hkv * sp.shares);
+  const int Hq = Hkv * G;
+  const int R = L * G;       // rows of a KV head
+  const int base = n - L;    // row i sees keys <= base + i
+
+  const int64_t row0 = ((int64_t)b * Hkv + hk) * cap;
+  const int last_row = n - 1;
+
+
+  // This workgroup's segments, one after the other: with SPLIT the parts of the blocks that its
+  // share of the KV head's tiles covers, else its one block whole (last position blocks first: they
+  // see the most keys, so the dispatch order is longest first). A variant of its own for whole
+  // blocks: the walk costs it 1.4% (2,048 rows at 82,671 keys, 2,486 -> 2,521 us).
+  int pb = SPLIT ? 0 : npb - 1 - share;
+  int u = sp.tiles * share;               // next tile, counted over the KV head's blocks in order
+  const int u_end = u + sp.tiles;
+  int u_blk = 0;                          // first tile of block pb in that count
+  if (SPLIT) {
+    int bt = prefill_tiles(pb, R, sp.g, base);
+    while (u >= u_blk + bt && pb < npb) {
+      u_blk += bt;
+      bt = prefill_tiles(++pb, R, sp.g, base);
+    }
+  }
+  for (bool more = !SPLIT || pb < npb; more;) {
+  // re-read per segment, so that no lane value derived from it is kept in registers across them
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
   const int lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool grp_a = wv < PW / 2;  // wave-uniform
   const int lc = lane & 15;
   const int lq4 = lane >> 4;
-  const int x = blockIdx.x;
-  const int hk = x % Hkv;  // consecutive workgroups (consecutive XCDs) take consecutive KV heads
-  // last position blocks first: they see the most keys, so the dispatch order is longest first
-  const int pb = npb - 1 - (x / Hkv) % npb;
-  const int b = x / (Hkv * npb);
-  const int Hq = Hkv * G;
-  const int R = L * G;       // rows of a KV head
-  const int base = n - L;    // row i sees keys <= base + i
-
+  const int T_blk = prefill_tiles(pb, R, sp.g, base);  // tiles the block needs
+  const int tb = SPLIT ? u - u_blk : 0;           // the segment: tiles tb .. tb + T - 1
+  const int T = SPLIT ? min(T_blk, u_end - u_blk) - tb : T_blk;
   // this wave's rows f0 .. f0 + 31 (row 16 nt + lc of the wave: f0 + 16 nt + lc)
   const int f0 = pb * PROWS + 32 * wv;
-  const int lim_lo = base + f0 / G;                                      // bound of its first row
-  const int lim_hi = f0 < R ? base + min(f0 + 31, R - 1) / G : -1;       // of its last valid row
-  const int wg_last = min(pb * PROWS + PROWS - 1, R - 1) / G;  // the workgroup's last position
-  const int T = (base + wg_last) / PT + 1;           // tiles the workgroup needs
-
-  const int64_t row0 = ((int64_t)b * Hkv + hk) * cap;
-  const int last_row = n - 1;
+  const int lim_lo = base + f0 / G;                                 // bound of its first row
+  const int lim_hi = f0 < R ? base + min(f0 + 31, R - 1) / G : -1;  // of its last valid row
 
   // ---- raw tile copies, per thread: two 16-byte K copies (wave wv: keys 16 wv .. 16 wv + 15),
   // two V copies, one word (wave wv: word array wv / 2, keys 64 (wv % 2) + lane)
@@ -169,7 +201,7 @@ __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
   const uint16_t* warr = wa == 0 ? ks : wa == 1 ? kb : wa == 2 ? vs : vb;
   const int wkey = 64 * (wv & 1) + lane;
   auto issue_codes = [&](int t, int slot) {
-    const int t0 = PT * min(t, T - 1);
+    const int t0 = PT * (tb + min(t, T - 1));
     const uint32_t lb = lds_raw + (uint32_t)slot * (uint32_t)sizeof(PrefillRaw);
     // M0 operands: wave-uniform values, made explicit so that they live in SGPRs
     const uint32_t mk = __builtin_amdgcn_readfirstlane(lb + offsetof(PrefillRaw, k) + 2048u * wv);
@@ -189,7 +221,7 @@ __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
     const uint32_t mw = __builtin_amdgcn_readfirstlane(
         lds_wd + (uint32_t)slot * (uint32_t)sizeof(PrefillWords) +
         4u * (uint32_t)(PT * wa + 64 * (wv & 1)));
-    const int64_t wr = row0 + min(PT * min(t, T - 1) + wkey, last_row);
+    const int64_t wr = row0 + min(PT * (tb + min(t, T - 1)) + wkey, last_row);
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off nt"
                  :: "v"(warr + wr * 2), "s"(mw) : "memory");
   };
@@ -579,7 +611,7 @@ __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
   // a tile ahead of the codes, so that a tile's range and factors are taken at the ends of the
   // matrix slots before it is dequantized (which the other half's vector phase outlasts) and not
   // in the dequantization slots, which set the pace: those made the loop 8% slower.
-  const int Tact = lim_hi < 0 ? 0 : min(T, lim_hi / PT + 1);
+  const int Tact = lim_hi < 0 ? 0 : max(0, min(T, lim_hi / PT + 1 - tb));
   int w0 = 0, w1 = 1;  // word slots of tiles t and t + 1
   auto next_words = [&]() {
     w0 = w1;
@@ -588,7 +620,7 @@ __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
   if (grp_a) {
     int t = 0;
     for (; t < Tact; ++t) {
-      const int t0 = PT * t;
+      const int t0 = PT * (tb + t);
       uint2 rw;                                         // slot 4t
       if (RANGE) rw = range_words(sm.wd[w1]);
       qk();
@@ -621,7 +653,7 @@ __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
   } else {
     int t = 0;
     for (; t < Tact; ++t) {
-      const int t0 = PT * t;
+      const int t0 = PT * (tb + t);
       dequant_v(sm.raw[t & 1], sm.wd[w0], kv);          // slot 4t
       __syncthreads();
       qk();                                             // slot 4t + 1
@@ -650,32 +682,152 @@ __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the clamped copies past the end
 
-  // ---- output rows: acc / l, V's factor taken out
+  // ---- output rows: acc / l, V's factor taken out; of a part of the block's tiles in fp32, with
+  // the row's (m, l), for prefill_merge_kernel
+  const bool whole = !SPLIT || T == T_blk;
+  const int64_t slot = 2 * (int64_t)x + (tb == 0);
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt) {
     const float l = lacc[nt][0];
-    if (lim[16 * nt] < 0) continue;
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    const int i = lim[16 * nt] - base, head = f0 + 16 * nt + lc - i * G;
-    uint16_t* orow = out + (((int64_t)b * Hq + hk * G + head) * L + i) * D;
+    const int last = lim[16 * nt];
+    if (last >= 0) {
+      const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+      const int wrow = 32 * wv + 16 * nt + lc;
+      const int i = last - base, head = pb * PROWS + wrow - i * G;
+      uint16_t* orow = out + (((int64_t)b * Hq + hk * G + head) * L + i) * D;
+      float* prow = sp.part_o + (slot * PROWS + wrow) * D;
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      f4_t o = oacc[nt][dt] * inv;
-      if (RANGE && kv_acc != 0) {  // wave-uniform, rare
+      for (int dt = 0; dt < 8; ++dt) {
+        f4_t o = oacc[nt][dt] * inv;
+        if (RANGE && kv_acc != 0) {  // wave-uniform, rare
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = ldexpf(o[r], kv_acc);
+          for (int r = 0; r < 4; ++r) o[r] = ldexpf(o[r], kv_acc);
+        }
+        if (whole) {
+          const uint32_t lo = (uint32_t)f32_to_bf16(o[0]) | ((uint32_t)f32_to_bf16(o[1]) << 16);
+          const uint32_t hi = (uint32_t)f32_to_bf16(o[2]) | ((uint32_t)f32_to_bf16(o[3]) << 16);
+          *reinterpret_cast<uint2*>(orow + 16 * dt + 4 * lq4) = make_uint2(lo, hi);
+        } else {
+          *reinterpret_cast<f4_t*>(prow + 16 * dt + 4 * lq4) = o;
+        }
       }
-      const uint32_t lo = (uint32_t)f32_to_bf16(o[0]) | ((uint32_t)f32_to_bf16(o[1]) << 16);
-      const uint32_t hi = (uint32_t)f32_to_bf16(o[2]) | ((uint32_t)f32_to_bf16(o[3]) << 16);
-      *reinterpret_cast<uint2*>(orow + 16 * dt + 4 * lq4) = make_uint2(lo, hi);
+      if (!whole && lq4 == 0) sp.part_ml[slot * PROWS + wrow] = make_float2(m_run[nt], l);
     }
   }
+
+  more = SPLIT && u_blk + T_blk < u_end && pb + 1 < npb;
+  u_blk += T_blk;
+  u = u_blk;
+  ++pb;
+  if (more) __syncthreads();  // the LDS is the next segment's
+  }
+}
+
+// Rows of split blocks: the shares' partial rows weighted by their sums (log-sum-exp). One
+// workgroup per 2 rows of a block; a row's parts (those of consecutive shares) are dealt to four
+// groups of 32 lanes (4 dims each), which combine through LDS. Blocks that one share covered whole
+// are written already. Bound by the loads' latency: 33 MB of parts (64 rows at 82,735 keys, 32/8
+// heads, 21 parts per row) took 20.4 us with one group per row and 8 rows per workgroup.
+__global__ __launch_bounds__(256) void prefill_merge_kernel(uint16_t* __restrict__ out, int n, int L,
+                                                            int Hkv, int G, PrefillSplit sp) {
+  __shared__ f4_t sh_acc[2][4][32];
+  __shared__ float2 sh_ml[2][4];
+  const int hk = blockIdx.y % Hkv, b = blockIdx.y / Hkv;
+  const int R = L * G, base = n - L;
+  const int pb = blockIdx.x / (PROWS / 2);
+  const int tr = threadIdx.x >> 7, grp = (threadIdx.x >> 5) & 3, ln = threadIdx.x & 31;
+  const int wrow = 2 * (blockIdx.x % (PROWS / 2)) + tr;
+  int u0 = 0;
+  for (int j = 0; j < pb; ++j) u0 += prefill_tiles(j, R, sp.g, base);
+  const int u1 = u0 + prefill_tiles(pb, R, sp.g, base);
+  const int j0 = u0 / sp.tiles, j1 = (u1 - 1) / sp.tiles;
+  const int f = pb * PROWS + wrow;
+  if (j0 == j1 || f - tr >= R) return;  // workgroup-uniform
+  const bool valid = f < R;
+  auto row = [&](int j) {  // row of share j's part of this block
+    const int64_t x = hk + (int64_t)Hkv * (j + (int64_t)sp.shares * b);
+    return (2 * x + (j == j0)) * PROWS + wrow;
+  };
+  float M = -INFINITY;
+  f4_t acc = {0.f, 0.f, 0.f, 0.f};
+  float den = 0.0f;
+  if (valid) {
+#pragma unroll 4
+    for (int j = j0 + grp; j <= j1; j += 4) M = fmaxf(M, sp.part_ml[row(j)].x);
+#pragma unroll 4
+    for (int j = j0 + grp; j <= j1; j += 4) {
+      const int64_t r = row(j);
+      const float2 ml = sp.part_ml[r];
+      const f4_t o = *reinterpret_cast<const f4_t*>(sp.part_o + r * D + 4 * ln);
+      const float w = ml.y > 0.0f ? exp2_nonpos(ml.x - M) * ml.y : 0.0f;
+      if (w > 0.0f) acc += o * w;
+      den += w;
+    }
+  }
+  sh_acc[tr][grp][ln] = acc;
+  if (ln == 0) sh_ml[tr][grp] = make_float2(M, den);
+  __syncthreads();
+  if (grp != 0 || !valid) return;
+  float mx = -INFINITY;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) mx = fmaxf(mx, sh_ml[tr][g].x);
+  acc = f4_t{0.f, 0.f, 0.f, 0.f};
+  den = 0.0f;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const float2 ml = sh_ml[tr][g];
+    const float w = ml.y > 0.0f ? exp2_nonpos(ml.x - mx) : 0.0f;
+    if (w > 0.0f) acc += sh_acc[tr][g][ln] * w;
+    den += w * ml.y;
+  }
+  const f4_t o = acc * (den > 0.0f ? 1.0f / den : 0.0f);
+  const int i = (int)fdiv_u((uint32_t)f, sp.g), head = f - i * G;
+  const uint32_t lo = (uint32_t)f32_to_bf16(o[0]) | ((uint32_t)f32_to_bf16(o[1]) << 16);
+  const uint32_t hi = (uint32_t)f32_to_bf16(o[2]) | ((uint32_t)f32_to_bf16(o[3]) << 16);
+  *reinterpret_cast<uint2*>(out + (((int64_t)b * Hkv * G + hk * G + head) * L + i) * D + 4 * ln) =
+      make_uint2(lo, hi);
+}
+
+// How the blocks of a chunk are dealt to workgroups: whole, one block each (tiles 0), or each KV
+// head's tiles, block after block, in equal shares of `tiles` for as many workgroups as fill the
+// CUs. Costs in tiles (3.7-4.2 us each, by clock): whole blocks go round by round, longest first;
+// a share pays about two per block that it touches (q, the first copies, the output rows) and the
+// partial rows with their merge launch about six. Measured, us per 32/8 chunk, whole against
+// split: 64 rows at 82,735 keys 2,068 / 137, 1,024 rows at 83,695 keys 2,138 / 1,440; 48/8, 512
+// rows at 8,193 keys, 237 / 147, 2,048 rows at 62,048 keys (1.5 rounds whole) 3,908 / 3,255; and
+// where whole stays better, 2,048 rows at 2,112 keys (17 tiles at most) 79 / 120.
+constexpr int SEGMENT_TILES = 2;
+constexpr int MERGE_TILES = 6;
+constexpr int MIN_SHARE = 4;
+PrefillSplit plan_split(int64_t B, int64_t Hkv, int64_t G, int64_t L, int64_t n, int cus) {
+  const int R = (int)(L * G), base = (int)(n - L), npb = (R + PROWS - 1) / PROWS;
+  PrefillSplit sp{make_fastdiv((uint32_t)G), npb, 0, nullptr, nullptr};
+  const int64_t S = cus / (B * Hkv);
+  if (S < 2 || npb > 4 * S) return sp;  // no CUs to spare; the last round matters little
+  int64_t total = 0, rounds = 0;
+  for (int pb = 0; pb < npb; ++pb) {
+    const int t = prefill_tiles(pb, R, sp.g, base);
+    total += t;
+    if ((npb - 1 - pb) % S == 0) rounds += t;
+  }
+  const int64_t tiles = std::max<int64_t>(MIN_SHARE, (total + S - 1) / S);
+  const int64_t touched = 2 + (tiles - 2) / prefill_tiles(0, R, sp.g, base);  // block 0: shortest
+  if (33 * (tiles + SEGMENT_TILES * touched + MERGE_TILES) > 32 * rounds) return sp;  // 3% or more
+  sp.tiles = (int)tiles;
+  sp.shares = (int)((total + tiles - 1) / tiles);
+  return sp;
+}
+
+int64_t split_bytes(const PrefillSplit& sp, int64_t B, int64_t Hkv) {
+  return sp.tiles ? 2 * B * Hkv * sp.shares * PROWS * (int64_t)(D * sizeof(float) + sizeof(float2))
+                  : 0;
 }
 
 int prefill_attn(const uint16_t* q, const uint8_t* kc, const uint16_t* ks, const uint16_t* kb,
                  const uint8_t* vc, const uint16_t* vs, const uint16_t* vb, int64_t B, int64_t Hq,
                  int64_t Hkv, int64_t L, int64_t D, int64_t cap, int64_t n, float scale,
-                 uint16_t* out, hipStream_t st) {
+                 uint16_t* out, bool split, void* workspace, int64_t workspace_bytes,
+                 hipStream_t st) {
   LQ_CHECK_ARG(D == 128, "head_dim must be 128 (got %lld)", (long long)D);
   LQ_CHECK_ARG(Hkv >= 1 && Hq >= Hkv && Hq % Hkv == 0, "Hq=%lld must be a multiple of Hkv=%lld",
                (long long)Hq, (long long)Hkv);
@@ -686,8 +838,20 @@ int prefill_attn(const uint16_t* q, const uint8_t* kc, const uint16_t* ks, const
                (long long)cap);
   LQ_CHECK_ARG(q && kc && ks && kb && vc && vs && vb && out, "null pointer");
   const int64_t npb = (L * G + PROWS - 1) / PROWS;
-  const int64_t wgs = B * Hkv * npb;
-  LQ_CHECK_ARG(wgs <= (int64_t)INT32_MAX, "too many workgroups");
+  LQ_CHECK_ARG(B * Hkv * npb <= (int64_t)INT32_MAX, "too many workgroups");
+  PrefillSplit sp{make_fastdiv((uint32_t)G), (int)npb, 0, nullptr, nullptr};
+  if (split) {
+    sp = plan_split(B, Hkv, G, L, n, device_cu_count());
+    const int64_t need = split_bytes(sp, B, Hkv);
+    if (need > 0 && (!workspace || workspace_bytes < need)) {
+      set_error("workspace of %lld bytes is smaller than the %lld needed",
+                (long long)workspace_bytes, (long long)need);
+      return LQ_EWORKSPACE;
+    }
+    sp.part_o = (float*)workspace;
+    sp.part_ml = (float2*)(sp.part_o + 2 * B * Hkv * sp.shares * PROWS * D);
+  }
+  const int64_t wgs = B * Hkv * sp.shares;
   // scores in log2 units; the range variant leaves q exact (bf16 times a power of two) and gives K,
   // which is rounded to fp16 anyway, the scale's mantissa in [0.5, 1)
   const float qk = scale * 1.4426950408889634f;
@@ -695,11 +859,17 @@ int prefill_attn(const uint16_t* q, const uint8_t* kc, const uint16_t* ks, const
   const float sm = std::frexp(qk, &se);
   // groupings that the verify kernel served before keep its range (see the top of the file)
   const bool range = !(G == 1 || G == 2 || G == 4 || G == 8);
-  (range ? q8_prefill_kernel<true> : q8_prefill_kernel<false>)<<<dim3((unsigned)wgs),
-                                                                 dim3(64 * PW), 0, st>>>(
+  auto* kern = range ? (sp.tiles ? q8_prefill_kernel<true, true> : q8_prefill_kernel<true, false>)
+                     : (sp.tiles ? q8_prefill_kernel<false, true> : q8_prefill_kernel<false, false>);
+  kern<<<dim3((unsigned)wgs), dim3(64 * PW), 0, st>>>(
       q, kc, ks, kb, vc, vs, vb, out, cap, (int)n, (int)L, (int)Hkv, (int)G, (int)npb,
-      range ? ldexpf(1.0f, se) : qk, range ? sm : 1.0f);
+      sp, range ? ldexpf(1.0f, se) : qk, range ? sm : 1.0f);
   LQ_CHECK_LAUNCH("q8_prefill_kernel");
+  if (sp.tiles) {
+    prefill_merge_kernel<<<dim3((unsigned)(npb * (PROWS / 2)), (unsigned)(B * Hkv)), dim3(256), 0,
+                           st>>>(out, (int)n, (int)L, (int)Hkv, (int)G, sp);
+    LQ_CHECK_LAUNCH("prefill_merge_kernel");
+  }
   return LQ_OK;
 }
 
@@ -717,8 +887,21 @@ extern "C" int lq_q8_prefill_attn(const uint16_t* q, const uint8_t* kc, const ui
                    Hq / Hkv == 8,
                "this entry takes 1, 2, 4 or 8 query heads per KV head (got %lld)",
                (long long)(Hq / Hkv));
-  return prefill_attn(q, kc, ks, kb, vc, vs, vb, B, Hq, Hkv, L, D, cap, n, scale, out,
-                      (hipStream_t)stream);
+  return prefill_attn(q, kc, ks, kb, vc, vs, vb, B, Hq, Hkv, L, D, cap, n, scale, out, false,
+                      nullptr, 0, (hipStream_t)stream);
+}
+
+extern "C" int64_t lq_prefill_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t L,
+                                              int64_t n) {
+  using namespace lq;
+  clear_error();
+  if (B < 1 || Hkv < 1 || Hq < Hkv || Hq % Hkv || Hq / Hkv > 64 || L < 1 || L > n ||
+      n > (1 << 24)) {
+    set_error("bad prefill shape B=%lld Hq=%lld Hkv=%lld L=%lld n=%lld", (long long)B,
+              (long long)Hq, (long long)Hkv, (long long)L, (long long)n);
+    return -1;
+  }
+  return split_bytes(plan_split(B, Hkv, Hq / Hkv, L, n, device_cu_count()), B, Hkv);
 }
 
 extern "C" int lq_q8_prefill_attn_grouped(const uint16_t* q, const uint8_t* kc, const uint16_t* ks,
@@ -726,8 +909,9 @@ extern "C" int lq_q8_prefill_attn_grouped(const uint16_t* q, const uint8_t* kc, 
                                           const uint16_t* vs, const uint16_t* vb, int64_t B,
                                           int64_t Hq, int64_t Hkv, int64_t L, int64_t D,
                                           int64_t cap, int64_t n, float scale, uint16_t* out,
+                                          void* workspace, int64_t workspace_bytes,
                                           void* stream) {
   lq::clear_error();
-  return lq::prefill_attn(q, kc, ks, kb, vc, vs, vb, B, Hq, Hkv, L, D, cap, n, scale, out,
-                          (hipStream_t)stream);
+  return lq::prefill_attn(q, kc, ks, kb, vc, vs, vb, B, Hq, Hkv, L, D, cap, n, scale, out, true,
+                          workspace, workspace_bytes, (hipStream_t)stream);
 }

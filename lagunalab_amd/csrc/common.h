@@ -64,6 +64,20 @@ int quantize_append(AppendTarget a, AppendTarget b, int two, int64_t B, int64_t 
                     int64_t D, int64_t cap, int64_t offset, int bits, int group_size,
                     hipStream_t st);
 
+// Unsigned division by a fixed divisor d >= 1 of values below 2^31: q = (mulhi(n, m) + n) >> l
+// with 2^(l-1) < d <= 2^l and m = floor(2^32 (2^l - d) / d) + 1 (Granlund and Montgomery, 1994).
+struct FastDiv {
+  uint32_t m, l;
+};
+inline FastDiv make_fastdiv(uint32_t d) {
+  uint32_t l = 0;
+  while ((1ull << l) < d) ++l;
+  return {(uint32_t)(((1ull << 32) * ((1ull << l) - d)) / d + 1), l};
+}
+__host__ __device__ __forceinline__ uint32_t fdiv_u(uint32_t n, FastDiv f) {
+  return ((uint32_t)(((uint64_t)n * f.m) >> 32) + n) >> f.l;
+}
+
 // ---------------------------------------------------------------------------------------------
 // device: number formats
 // ---------------------------------------------------------------------------------------------

@@ -17,21 +17,6 @@
 namespace lq {
 namespace {
 
-// Unsigned division by a fixed divisor d >= 1 of values below 2^31: q = (mulhi(n, m) + n) >> l
-// with 2^(l-1) < d <= 2^l and m = floor(2^32 (2^l - d) / d) + 1 (Granlund and Montgomery, 1994).
-struct FastDiv {
-  uint32_t m, l;
-};
-FastDiv make_fastdiv(uint32_t d) {
-  uint32_t l = 0;
-  while ((1ull << l) < d) ++l;
-  const uint64_t m = ((1ull << 32) * ((1ull << l) - d)) / d + 1;
-  return {(uint32_t)m, l};
-}
-__device__ __forceinline__ uint32_t fdiv_u(uint32_t n, FastDiv f) {
-  return (__umulhi(n, f.m) + n) >> f.l;
-}
-
 // Code of one value: round-half-away(fl(fl(x - bias) / scale)) clamped to 2^BITS - 1, as
 // affine_code. Fast path: u = (x - bias) * (1 / scale) + 0.5 (v_rcp_f32, 1 ulp) is within
 // 6.1e-5 of fl(fl(x - bias) / scale) + 0.5 for quotients below 512 (ours stay below 257), so

@@ -403,10 +403,15 @@ def q8_prefill_attention(q, keys, values, n, scale):
     if not L <= int(n) <= cap:
         raise ValueError(f"n={n} must cover the {L} chunk rows and fit the capacity {cap}")
     out = torch.empty((B, Hq, L, D), dtype=torch.bfloat16, device=dev)
+    ws_bytes = lib.lq_prefill_workspace_bytes(B, Hq, Hkv, L, int(n))
+    if ws_bytes < 0:
+        raise ValueError(lib.lq_last_error().decode())
+    # partial rows of a split chunk: tens of MB, so back to the allocator after the call
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
     st = lib.lq_q8_prefill_attn_grouped(qb.data_ptr(), kc.data_ptr(), ks.data_ptr(), kb.data_ptr(),
                                         vc.data_ptr(), vs.data_ptr(), vb.data_ptr(), B, Hq, Hkv, L,
-                                        D, cap, int(n), float(scale), out.data_ptr(),
-                                        _lib.stream_ptr(dev))
+                                        D, cap, int(n), float(scale), out.data_ptr(), _lib.ptr(ws),
+                                        ws_bytes, _lib.stream_ptr(dev))
     _lib.check(st, "lq_q8_prefill_attn_grouped")
     return out.to(q.dtype)
 

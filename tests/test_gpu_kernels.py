@@ -902,3 +902,46 @@ def test_prefill_of_any_grouping_matches_the_blocked_path(dev, n, L, G, Hkv, B):
                       "against the blocked path")
     assert_attn_close(got, A.fused_attention(q, cache_np(kq), cache_np(vq), n, 0.09, causal=True),
                       "against the oracle")
+
+
+@pytest.mark.parametrize("n,L,G,Hkv,B", [(9000, 20, 6, 2, 1), (3001, 300, 4, 2, 2), (20000, 17, 64, 1, 1),
+                                         (4700, 600, 1, 1, 1), (6000, 40, 4, 8, 1),
+                                         (2560, 600, 5, 1, 3)])
+def test_prefill_split_over_the_keys(dev, n, L, G, Hkv, B):
+    """Chunks of few blocks have their keys split: shares that end inside blocks, and parts in which
+    rows see no key. Against the float64 oracle; the workspace is needed and may hold anything, NaN
+    here."""
+    from lagunalab_amd import _lib, q8_attn
+    lib = _lib.load()
+    need = lib.lq_prefill_workspace_bytes(B, Hkv * G, Hkv, L, n)
+    assert need > 0
+    rng = np.random.default_rng(n + L + G)
+    kq, vq = make_cache(rng, B, Hkv, n, n + 3, dev)
+    q = Q.randn_bf16(rng, (B, Hkv * G, L, 128))
+    qd = to_dev_bf16(q, dev)
+    want = A.fused_attention(q, cache_np(kq), cache_np(vq), n, 0.09, causal=True)
+    assert_attn_close(q8_attn.q8_prefill_attention(qd, kq, vq, n, 0.09), want, "split")
+    ws = torch.full((need // 4,), float("nan"), device=dev)
+    out = torch.empty_like(qd)
+    args = [qd.data_ptr(), *(t.data_ptr() for t in (*kq, *vq)), B, Hkv * G, Hkv, L, 128, n + 3, n, 0.09,
+            out.data_ptr(), ws.data_ptr()]
+    assert lib.lq_q8_prefill_attn_grouped(*args, need - 1, None) == _lib.LQ_EWORKSPACE
+    assert lib.lq_q8_prefill_attn_grouped(*args, need, _lib.stream_ptr(dev)) == _lib.LQ_OK
+    assert_attn_close(out, want, "split, workspace of NaN")
+
+
+def test_prefill_split_shares_cover_several_blocks(dev):
+    """25 blocks per KV head on 10 workgroups each: shares of two and a half blocks (the end of one,
+    a whole one, the start of the next), against the entry that never splits."""
+    from lagunalab_amd import _lib, q8_attn
+    lib = _lib.load()
+    n, L, G, Hkv, B = 6600, 1600, 4, 8, 3
+    rng = np.random.default_rng(3)
+    kq, vq = make_cache(rng, B, Hkv, n, n, dev)
+    q = to_dev_bf16(Q.randn_bf16(rng, (B, Hkv * G, L, 128)), dev)
+    assert lib.lq_prefill_workspace_bytes(B, Hkv * G, Hkv, L, n) > 0
+    got = q8_attn.q8_prefill_attention(q, kq, vq, n, 0.09)
+    want = torch.empty_like(q)
+    assert lib.lq_q8_prefill_attn(q.data_ptr(), *(t.data_ptr() for t in (*kq, *vq)), B, Hkv * G, Hkv,
+                                  L, 128, n, n, 0.09, want.data_ptr(), _lib.stream_ptr(dev)) == 0
+    assert_attn_close(got, want.float().cpu().numpy(), "split against whole blocks")
