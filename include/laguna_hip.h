@@ -78,6 +78,12 @@ int lq_dequantize(const uint8_t* codes, const uint16_t* scales, const uint16_t* 
                   int64_t B, int64_t H, int64_t cap, int64_t n, int64_t D, int bits,
                   int group_size, uint16_t* out, void* stream);
 
+/* lq_dequantize of the keys and of the values of one cache in a single launch. */
+int lq_dequantize_kv(const uint8_t* k_codes, const uint16_t* k_scales, const uint16_t* k_biases,
+                     const uint8_t* v_codes, const uint16_t* v_scales, const uint16_t* v_biases,
+                     int64_t B, int64_t H, int64_t cap, int64_t n, int64_t D, int bits,
+                     int group_size, uint16_t* k_out, uint16_t* v_out, void* stream);
+
 /*
  * Scratch bytes for lq_decode_attn with the same B / Hq / Hkv / lengths. `lens_host` (host, B
  * entries) may be NULL, then every sequence has length n. Returns a negative value on bad args.

@@ -29,6 +29,8 @@ SIGNATURES = {
     "lq_quantize_append_kv": (i32, [vp, vp, i64, i64, i64, i64, vp, vp, vp, vp, vp, vp, i64, i64,
                                     i32, i32, vp]),
     "lq_dequantize": (i32, [vp, vp, vp, i64, i64, i64, i64, i64, i32, i32, vp, vp]),
+    "lq_dequantize_kv": (i32, [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i32, i32, vp, vp,
+                               vp]),
     "lq_decode_workspace_bytes": (i64, [i32, i64, i64, i64, i64, i64, vp]),
     "lq_decode_attn": (i32, [i32, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, vp,
                              f32, vp, vp, i64, vp]),

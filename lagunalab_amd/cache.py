@@ -25,7 +25,7 @@ from __future__ import annotations
 
 import torch
 
-from .quant import dequantize, quantize_kv_into
+from .quant import dequantize_kv, quantize_kv_into
 
 
 def create_attention_mask(N: int, offset: int = 0, return_array: bool = False,
@@ -212,9 +212,8 @@ class DequantKVCache:
         self._quantized_step = self.quantized_decode and L == 1
         if self._quantized_step:
             return qk, qv
-        g, b = self.q.group_size, self.q.bits
-        n = self.q.offset
-        return dequantize(*self.q.keys, g, b, n=n), dequantize(*self.q.values, g, b, n=n)
+        return dequantize_kv(self.q.keys, self.q.values, self.q.group_size, self.q.bits,
+                             self.q.offset)
 
     def attend(self, queries, scale):
         """Attention straight off the packed cache: the fused decode kernel for one query row,

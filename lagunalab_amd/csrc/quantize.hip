@@ -156,47 +156,89 @@ __global__ __launch_bounds__(256) void quantize_group_kernel(
   }
 }
 
-// One thread per 8 consecutive elements of one row (8 divides every group size).
+// The first n rows of every head, of one or two caches of one shape (K and V in one launch). A
+// head's rows are contiguous on both sides, so element e of a head's n x D is element e of its
+// output and a workgroup needs one division (its head); a thread takes DQ_ITER runs of 8 elements
+// (8 divides every group size), 256 runs apart, all loads before the first store. Bound by its traffic: a
+// token's append and 32,769 rows x 8 heads x 128 of K and V (205 MB read and written; a large copy runs at 4.7-5.2
+// TB/s) take 49 us, with a launch each, 64-bit divisions per run and one run per thread 56.
+constexpr int DQ_ITER = 4;
+struct DequantTarget {
+  const uint8_t* codes;
+  const uint16_t* scales;
+  const uint16_t* biases;
+  uint16_t* out;
+};
+
 template <int BITS>
-__global__ __launch_bounds__(256) void dequantize_kernel(
-    const uint8_t* __restrict__ codes, const uint16_t* __restrict__ scales,
-    const uint16_t* __restrict__ biases, int64_t BH, int64_t cap, int64_t n, int D, int gs,
-    uint16_t* __restrict__ out) {
-  const int64_t per_row = D / 8;
-  const int64_t total = BH * n * per_row;
-  const int groups_per_row = D / gs;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = i / per_row;  // output row in [BH * n)
-    const int d0 = (int)(i - r * per_row) * 8;
-    const int64_t bh = r / n;
-    const int64_t t = r - bh * n;
-    const int64_t crow = bh * cap + t;
-    const int gr = d0 / gs;
-    const float s = bf16_to_f32(scales[crow * groups_per_row + gr]);
-    const float b = bf16_to_f32(biases[crow * groups_per_row + gr]);
-    uint32_t cv[8];
-    if (BITS == 8) {
-      const uint2 w = *reinterpret_cast<const uint2*>(codes + crow * D + d0);
+__global__ __launch_bounds__(256) void dequantize_kernel(DequantTarget ta, DequantTarget tb,
+                                                         uint32_t wgs_per_head, uint32_t BH,
+                                                         int64_t head_in, int64_t head_out,
+                                                         int gs_shift) {
+  uint32_t hd = blockIdx.x / wgs_per_head;
+  const int64_t e0 = ((int64_t)(blockIdx.x - hd * wgs_per_head) * (256 * DQ_ITER) + threadIdx.x) * 8;
+  const bool second = hd >= BH;  // workgroup-uniform
+  if (second) hd -= BH;
+  const DequantTarget t = second ? tb : ta;
+  const int64_t in0 = hd * head_in;  // elements before this head's rows
+  const uint8_t* codes = t.codes + in0 * BITS / 8;
+  const uint16_t* scales = t.scales + (in0 >> gs_shift);
+  const uint16_t* biases = t.biases + (in0 >> gs_shift);
+  uint16_t* out = t.out + hd * head_out;
+  uint2 w[DQ_ITER];
+  uint16_t sc[DQ_ITER], bi[DQ_ITER];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        cv[k] = (w.x >> (8 * k)) & 0xffu;
-        cv[4 + k] = (w.y >> (8 * k)) & 0xffu;
-      }
-    } else {
-      const uint32_t w = *reinterpret_cast<const uint32_t*>(codes + crow * (D / 2) + d0 / 2);
+  for (int k = 0; k < DQ_ITER; ++k) {
+    const int64_t e = e0 + k * (256 * 8);
+    if (e >= head_out) continue;
+    if (BITS == 8) w[k] = *reinterpret_cast<const uint2*>(codes + e);
+    else w[k].x = *reinterpret_cast<const uint32_t*>(codes + e / 2);
+    sc[k] = scales[e >> gs_shift];
+    bi[k] = biases[e >> gs_shift];
+  }
 #pragma unroll
-      for (int k = 0; k < 8; ++k) cv[k] = (w >> (4 * k)) & 0xfu;
-    }
+  for (int k = 0; k < DQ_ITER; ++k) {
+    const int64_t e = e0 + k * (256 * 8);
+    if (e >= head_out) continue;
+    const float s = bf16_to_f32(sc[k]), b = bf16_to_f32(bi[k]);
     uint32_t o[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint16_t a = f32_to_bf16(__fadd_rn(__fmul_rn(s, (float)cv[2 * k]), b));
-      const uint16_t c = f32_to_bf16(__fadd_rn(__fmul_rn(s, (float)cv[2 * k + 1]), b));
-      o[k] = (uint32_t)a | ((uint32_t)c << 16);
+    for (int j = 0; j < 4; ++j) {
+      uint32_t c0, c1;
+      if (BITS == 8) {
+        const uint32_t x = (j < 2 ? w[k].x : w[k].y) >> (16 * (j & 1));
+        c0 = x & 0xffu;
+        c1 = (x >> 8) & 0xffu;
+      } else {
+        c0 = (w[k].x >> (8 * j)) & 0xfu;
+        c1 = (w[k].x >> (8 * j + 4)) & 0xfu;
+      }
+      o[j] = (uint32_t)f32_to_bf16(__fadd_rn(__fmul_rn(s, (float)c0), b)) |
+             ((uint32_t)f32_to_bf16(__fadd_rn(__fmul_rn(s, (float)c1), b)) << 16);
     }
-    *reinterpret_cast<uint4*>(out + r * D + d0) = make_uint4(o[0], o[1], o[2], o[3]);
+    *reinterpret_cast<uint4*>(out + e) = make_uint4(o[0], o[1], o[2], o[3]);
   }
+}
+
+int dequantize(DequantTarget a, DequantTarget b, int two, int64_t B, int64_t H, int64_t cap,
+               int64_t n, int64_t D, int bits, int group_size, hipStream_t st) {
+  LQ_CHECK_ARG(bits == 4 || bits == 8, "bits must be 4 or 8 (got %d)", bits);
+  LQ_CHECK_ARG(group_size == 32 || group_size == 64 || group_size == 128,
+               "group_size must be 32, 64 or 128 (got %d)", group_size);
+  LQ_CHECK_ARG(B >= 1 && H >= 1 && D >= 1 && D % group_size == 0, "bad shape");
+  LQ_CHECK_ARG(n >= 0 && n <= cap, "n=%lld outside [0, cap=%lld]", (long long)n, (long long)cap);
+  LQ_CHECK_ARG(a.codes && a.scales && a.biases && a.out, "null pointer");
+  LQ_CHECK_ARG(!two || (b.codes && b.scales && b.biases && b.out), "null pointer");
+  if (n == 0) return LQ_OK;
+  const int64_t per_head = (n * D / 8 + 256 * DQ_ITER - 1) / (256 * DQ_ITER);
+  const int64_t wgs = (two ? 2 : 1) * B * H * per_head;
+  LQ_CHECK_ARG(wgs < (int64_t)1 << 31, "dequantization of %lld values is too large for one call",
+               (long long)(B * H * n * D));
+  const int shift = group_size == 32 ? 5 : group_size == 64 ? 6 : 7;
+  (bits == 8 ? dequantize_kernel<8> : dequantize_kernel<4>)<<<dim3((unsigned)wgs), dim3(256), 0, st>>>(
+      a, b, (uint32_t)per_head, (uint32_t)(B * H), cap * D, n * D, shift);
+  LQ_CHECK_LAUNCH("dequantize_kernel");
+  return LQ_OK;
 }
 
 template <int BITS, int GS>
@@ -273,20 +315,18 @@ extern "C" int lq_dequantize(const uint8_t* codes, const uint16_t* scales, const
                              int group_size, uint16_t* out, void* stream) {
   using namespace lq;
   clear_error();
-  LQ_CHECK_ARG(bits == 4 || bits == 8, "bits must be 4 or 8 (got %d)", bits);
-  LQ_CHECK_ARG(group_size == 32 || group_size == 64 || group_size == 128,
-               "group_size must be 32, 64 or 128 (got %d)", group_size);
-  LQ_CHECK_ARG(B >= 1 && H >= 1 && D >= 1 && D % group_size == 0, "bad shape");
-  LQ_CHECK_ARG(n >= 0 && n <= cap, "n=%lld outside [0, cap=%lld]", (long long)n, (long long)cap);
-  LQ_CHECK_ARG(codes && scales && biases && out, "null pointer");
-  if (n == 0) return LQ_OK;
-  const int64_t total = B * H * n * (D / 8);
-  const int64_t blocks = std::min<int64_t>((total + 255) / 256, 65536);
-  hipStream_t st = (hipStream_t)stream;
-  if (bits == 8)
-    dequantize_kernel<8><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(codes, scales, biases, B * H, cap, n, (int)D, group_size, out);
-  else
-    dequantize_kernel<4><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(codes, scales, biases, B * H, cap, n, (int)D, group_size, out);
-  LQ_CHECK_LAUNCH("dequantize_kernel");
-  return LQ_OK;
+  const DequantTarget a{codes, scales, biases, out};
+  return dequantize(a, a, 0, B, H, cap, n, D, bits, group_size, (hipStream_t)stream);
+}
+
+extern "C" int lq_dequantize_kv(const uint8_t* k_codes, const uint16_t* k_scales,
+                                const uint16_t* k_biases, const uint8_t* v_codes,
+                                const uint16_t* v_scales, const uint16_t* v_biases, int64_t B,
+                                int64_t H, int64_t cap, int64_t n, int64_t D, int bits,
+                                int group_size, uint16_t* k_out, uint16_t* v_out, void* stream) {
+  using namespace lq;
+  clear_error();
+  const DequantTarget a{k_codes, k_scales, k_biases, k_out};
+  const DequantTarget b{v_codes, v_scales, v_biases, v_out};
+  return dequantize(a, b, 1, B, H, cap, n, D, bits, group_size, (hipStream_t)stream);
 }

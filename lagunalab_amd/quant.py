@@ -115,3 +115,27 @@ def dequantize(codes: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                            group_size, out.data_ptr(), _lib.stream_ptr(dev))
     _lib.check(st, "lq_dequantize")
     return out
+
+
+def dequantize_kv(kbuf, vbuf, group_size: int, bits: int, n: int):
+    """:func:`dequantize` of rows ``[0, n)`` of a cache's keys and values (``(codes, scales,
+    biases)`` tuples of uint8 codes), in one launch when their shapes agree."""
+    kc, ks, kb = kbuf
+    vc, vs, vb = vbuf
+    if not (kc.shape == vc.shape and ks.shape == kb.shape == vs.shape == vb.shape and n
+            and all(t.is_contiguous() for t in (*kbuf, *vbuf))
+            and kc.dtype == vc.dtype == torch.uint8
+            and all(t.dtype == torch.bfloat16 for t in (ks, kb, vs, vb))):
+        return dequantize(kc, ks, kb, group_size, bits, n=n), dequantize(vc, vs, vb, group_size, bits, n=n)
+    lib = _lib.load()
+    _check_bits(bits, group_size)
+    dev = _lib.require_device(*kbuf, *vbuf)
+    B, H, cap, nb = kc.shape
+    D = nb * 8 // bits
+    k = torch.empty((B, H, n, D), dtype=torch.bfloat16, device=dev)
+    v = torch.empty((B, H, n, D), dtype=torch.bfloat16, device=dev)
+    st = lib.lq_dequantize_kv(kc.data_ptr(), ks.data_ptr(), kb.data_ptr(), vc.data_ptr(),
+                              vs.data_ptr(), vb.data_ptr(), B, H, cap, n, D, bits, group_size,
+                              k.data_ptr(), v.data_ptr(), _lib.stream_ptr(dev))
+    _lib.check(st, "lq_dequantize_kv")
+    return k, v

@@ -945,3 +945,29 @@ def test_prefill_split_shares_cover_several_blocks(dev):
     assert lib.lq_q8_prefill_attn(q.data_ptr(), *(t.data_ptr() for t in (*kq, *vq)), B, Hkv * G, Hkv,
                                   L, 128, n, n, 0.09, want.data_ptr(), _lib.stream_ptr(dev)) == 0
     assert_attn_close(got, want.float().cpu().numpy(), "split against whole blocks")
+
+
+@pytest.mark.parametrize("bits,gs,D,n,cap,B,H", [(8, 64, 128, 1, 4, 1, 1), (8, 64, 128, 65, 65, 2, 3),
+                                                 (4, 64, 128, 64, 100, 1, 2), (8, 32, 96, 21, 30, 1, 5),
+                                                 (4, 128, 128, 513, 600, 1, 2), (8, 64, 64, 1025, 1030, 1, 1)])
+def test_dequantize_kv_bit_exact(dev, bits, gs, D, n, cap, B, H):
+    """K and V dequantized in one launch: head lengths around a workgroup's 8,192 elements, ragged
+    against the capacity; equal to the oracle's bf16(scale * code + bias) bit for bit."""
+    from lagunalab_amd.quant import dequantize, dequantize_kv, quantize_into
+    rng = np.random.default_rng(n + D)
+    bufs = []
+    for _ in range(2):
+        c = (torch.zeros((B, H, cap, D * bits // 8), dtype=torch.uint8, device=dev),
+             torch.zeros((B, H, cap, D // gs), dtype=torch.bfloat16, device=dev),
+             torch.zeros((B, H, cap, D // gs), dtype=torch.bfloat16, device=dev))
+        quantize_into(to_dev_bf16(Q.randn_bf16(rng, (B, H, cap, D)), dev), *c, 0, gs, bits)
+        bufs.append(c)
+    k, v = dequantize_kv(*bufs, gs, bits, n)
+    for got, buf in ((k, bufs[0]), (v, bufs[1])):
+        codes, s, b = (t[:, :, :n] for t in buf)
+        if bits == 4:
+            codes = torch.stack([codes & 15, codes >> 4], -1).reshape(B, H, n, D)
+        want = (codes.float() * s.float().repeat_interleave(gs, -1)
+                + b.float().repeat_interleave(gs, -1)).to(torch.bfloat16)
+        assert torch.equal(got, want)
+        assert torch.equal(dequantize(*buf, gs, bits, n=n), want)
