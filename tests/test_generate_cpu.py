@@ -101,3 +101,32 @@ def test_greedy_stops_at_eos(model):
     free = generate_greedy(model, prompt, 6)
     got = generate_greedy(model, prompt, 6, eos=(free[2],))
     assert got == free[:free.index(free[2]) + 1]
+
+
+def test_pending_rows_behave_as_the_tuple_of_views():
+    """The tuple of a fused step makes its views on first use: every way of reading it completes the
+    append first and gives the views of the step's own buffers and length, also after the cache has
+    grown or been trimmed."""
+    import copy
+    from lagunalab_amd.cache import _PendingRows
+
+    class Cache:
+        flushed = 0
+
+        def _flush(self):
+            self.flushed += 1
+
+    bufs = tuple(torch.arange(24.).reshape(1, 2, 4, 3) + i for i in range(3))
+    want = tuple(t[:, :, :3] for t in bufs)
+    same = lambda a, b: len(a) == len(b) and all(torch.equal(x, y) for x, y in zip(a, b))  # noqa: E731
+    reads = [tuple, list, lambda p: [p[0], p[1], p[-1]], lambda p: [*p], lambda p: p[:],
+             lambda p: (lambda *a: a)(*p), lambda p: list(reversed(p))[::-1], lambda p: p + (),
+             lambda p: () + p, lambda p: p * 1, copy.copy, lambda p: (lambda a, b, c: (a, b, c))(*p)]
+    for read in reads:
+        c = Cache()
+        p = _PendingRows(bufs, 3, c)
+        assert isinstance(p, tuple) and len(p) == 3 and c.flushed == 0
+        assert same(read(p), want) and c.flushed > 0
+    p = _PendingRows(bufs, 3, Cache())
+    assert p == p and p[0] is p[0] and p[0] in p and p.index(p[0]) == 0 and hash(p) == hash(tuple(p))
+    assert "tensor" in repr(p)
