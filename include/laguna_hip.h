@@ -250,6 +250,23 @@ int lq_qk_norm_rope(const uint16_t* q, const uint16_t* k, uint16_t* q_out, uint1
 int lq_gate_heads(const uint16_t* attn, const uint16_t* gate, uint16_t* out, int64_t B,
                   int64_t Hq, int64_t L, int64_t D, int per_dim, void* stream);
 
+/* lq_gate_heads with the gate of row (b, l) at gate + (b L + l) gate_stride (a column range of wider
+ * rows, such as a block's projection; a per-dim gate 16-byte aligned, its stride a multiple of 8). */
+int lq_gate_heads_strided(const uint16_t* attn, const uint16_t* gate, int64_t gate_stride,
+                          uint16_t* out, int64_t B, int64_t Hq, int64_t L, int64_t D, int per_dim,
+                          void* stream);
+
+/*
+ * lq_qk_norm_rope from a block's projection rows proj [B, L, N] (q heads, k heads, v heads, then
+ * anything), which also takes them apart: q_out bf16 [B, Hq, L, 128] and k_out [B, Hkv, L, 128]
+ * normalized and rotated, v_out [B, Hkv, L, 128] as projected. Rows 4-byte aligned when N is even.
+ */
+int lq_qkv_norm_rope(const uint16_t* proj, int64_t N, uint16_t* q_out, uint16_t* k_out,
+                     uint16_t* v_out, const uint16_t* q_norm_w, const uint16_t* k_norm_w,
+                     int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t D, float eps,
+                     const float* inv_freq, int64_t rot_dims, float mscale, int64_t offset,
+                     void* stream);
+
 /*
  * Residual add + RMSNorm of a decoder layer's input (laguna.py's input_layernorm after the
  * previous block's residual add): h_out = h + d (bf16; d may be null: no add, h_out unused),

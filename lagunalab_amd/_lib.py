@@ -47,6 +47,9 @@ SIGNATURES = {
     "lq_greedy_accept": (i32, [vp, i64, i64, vp, i64, vp, vp, i64, vp]),
     "lq_qk_norm_rope": (i32, [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, f32, vp, i64, f32,
                               i64, vp, vp]),
+    "lq_qkv_norm_rope": (i32, [vp, i64, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, f32, vp, i64, f32,
+                               i64, vp]),
+    "lq_gate_heads_strided": (i32, [vp, vp, i64, vp, i64, i64, i64, i64, i32, vp]),
     "lq_gate_heads": (i32, [vp, vp, vp, i64, i64, i64, i64, i32, vp]),
     "lq_add_rms_norm": (i32, [vp, vp, vp, vp, vp, i64, i64, f32, vp]),
     "lq_gemv_bf16": (i32, [vp, vp, vp, i64, i64, vp]),

@@ -10,10 +10,11 @@ mlx-lm's SDPA routes it), SDPA over the returned K/V otherwise, then the softplu
 * one GEMM for q, k, v and the gate logits (the four projection weights concatenated), one for
   ``o_proj``: ``lq_gemv_bf16`` for a single row (a decode step), hipBLASLt through torch for
   more rows;
-* ``lq_qk_norm_rope``: the q and k RMSNorms and the rotary embedding of both in one launch
+* ``lq_qkv_norm_rope``: the projection taken apart, the q and k RMSNorms and the rotary embedding
+  of both in one launch
   (frequencies from :func:`rope_frequencies`: mlx-lm's default or YaRN RoPE, partial rotary);
 * the cache: the fused decode / verify kernels, or dequantized K/V for the unfused path;
-* ``lq_gate_heads``: softplus gate times the attention output, written in ``o_proj``'s layout.
+* ``lq_gate_heads_strided``: softplus gate times the attention output, written in ``o_proj``'s layout.
 
 Activations and weights are bf16, as in the reference's MLX model.
 """
@@ -131,17 +132,16 @@ class Attention:
         H, Hkv, D = self.n_heads, self.n_kv_heads, self.head_dim
         x = x.to(torch.bfloat16)
         proj = linear(x, self.w_in)  # [B, L, (H + 2 Hkv) D + gate]
-        qp, kp, vp, gp = torch.split(proj, self._splits, dim=-1)
-        q = qp.reshape(B, L, H, D).transpose(1, 2).contiguous()
-        k = kp.reshape(B, L, Hkv, D).transpose(1, 2).contiguous()
-        v = vp.reshape(B, L, Hkv, D).transpose(1, 2).contiguous()
-        g = gp.contiguous()
+        N = proj.shape[-1]
+        q = torch.empty((B, H, L, D), dtype=torch.bfloat16, device=dev)
+        k = torch.empty((B, Hkv, L, D), dtype=torch.bfloat16, device=dev)
+        v = torch.empty((B, Hkv, L, D), dtype=torch.bfloat16, device=dev)
         offset = cache.offset if cache is not None else 0
-        _lib.check(lib.lq_qk_norm_rope(q.data_ptr(), k.data_ptr(), q.data_ptr(), k.data_ptr(),
-                                       self.q_norm.data_ptr(), self.k_norm.data_ptr(), B, H, Hkv,
-                                       L, D, self.eps, self.inv_freq.data_ptr(), self.rot_dims,
-                                       self.mscale, int(offset), None, _lib.stream_ptr(dev)),
-                   "lq_qk_norm_rope")
+        _lib.check(lib.lq_qkv_norm_rope(proj.data_ptr(), N, q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                        self.q_norm.data_ptr(), self.k_norm.data_ptr(), B, H, Hkv,
+                                        L, D, self.eps, self.inv_freq.data_ptr(), self.rot_dims,
+                                        self.mscale, int(offset), _lib.stream_ptr(dev)),
+                   "lq_qkv_norm_rope")
         if cache is not None:
             k, v = cache.update_and_fetch(k, v)
         if getattr(cache, "fused_step", False):
@@ -154,7 +154,8 @@ class Attention:
             out = _sdpa(q, k, v, mask, self.scale)
         out = out.to(torch.bfloat16).contiguous()
         y = torch.empty((B, L, H, D), dtype=torch.bfloat16, device=dev)
-        _lib.check(lib.lq_gate_heads(out.data_ptr(), g.data_ptr(), y.data_ptr(), B, H, L, D,
-                                     0 if self.per_head_gate else 1, _lib.stream_ptr(dev)),
-                   "lq_gate_heads")
+        gate = proj.data_ptr() + 2 * (H + 2 * Hkv) * D  # the last columns of the projection rows
+        _lib.check(lib.lq_gate_heads_strided(out.data_ptr(), gate, N, y.data_ptr(), B, H, L, D,
+                                             0 if self.per_head_gate else 1, _lib.stream_ptr(dev)),
+                   "lq_gate_heads_strided")
         return linear(y.reshape(B, L, H * D), self.wo)

@@ -46,13 +46,45 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
                      mscale, pos);
 }
 
+// The same from the raw projection rows proj [B, L, N] of a block (q heads, k heads, v heads, then
+// the gate): one wave per (row, head), neighbouring waves on neighbouring heads of a row, q and k
+// normalized and rotated, v moved, each into its [B, H, L, 128] layout. The four strided pieces
+// were copied out by a launch each before (8 rows, 32/8 heads: 16 us of GPU time in five launches,
+// 3.5 us in this one). N may be odd (a per-head gate of odd Hq): then rows are read by 16 bits.
+__global__ __launch_bounds__(256) void qkv_norm_rope_kernel(
+    const uint16_t* __restrict__ proj, int64_t N, uint16_t* __restrict__ q_out,
+    uint16_t* __restrict__ k_out, uint16_t* __restrict__ v_out, const uint16_t* __restrict__ q_w,
+    const uint16_t* __restrict__ k_w, int64_t rows, int Hq, int Hkv, int64_t L, float eps,
+    const float* __restrict__ inv_freq, int rot_dims, float mscale, int64_t offset) {
+  const int lane = threadIdx.x & 63;
+  const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);  // over B L (Hq + 2 Hkv)
+  const int heads = Hq + 2 * Hkv;
+  const int64_t row = item / heads;
+  if (row >= rows) return;  // wave-uniform
+  const int hd = (int)(item - row * heads);
+  const int64_t b = row / L, l = row - b * L;
+  const uint16_t* in = proj + row * N + (int64_t)hd * ND + 2 * lane;
+  const uint32_t x = (N & 1) == 0 ? *reinterpret_cast<const uint32_t*>(in)
+                                  : (uint32_t)in[0] | ((uint32_t)in[1] << 16);
+  if (hd >= Hq + Hkv) {
+    reinterpret_cast<uint32_t*>(v_out + ((b * Hkv + hd - Hq - Hkv) * L + l) * ND)[lane] = x;
+    return;
+  }
+  const bool is_q = hd < Hq;
+  uint16_t* out = is_q ? q_out + ((b * Hq + hd) * L + l) * ND
+                       : k_out + ((b * Hkv + hd - Hq) * L + l) * ND;
+  reinterpret_cast<uint32_t*>(out)[lane] =
+      norm_rope_lane(x, reinterpret_cast<const uint32_t*>(is_q ? q_w : k_w)[lane], lane, eps,
+                     inv_freq, rot_dims, mscale, (float)(offset + l));
+}
+
 // softplus(x) = log(1 + e^x), written as max(x, 0) + log1p(e^-|x|) (no overflow for large x)
 __device__ __forceinline__ float softplus_f(float x) { return fmaxf(x, 0.0f) + log1pf(expf(-fabsf(x))); }
 
-// One thread per 8 dims of one (b, h, l) row of attn [B, Hq, L, D]; gate g is [B, L, Hq] (per
-// head) or [B, L, Hq, D] (per dim).
+// One thread per 8 dims of one (b, h, l) row of attn [B, Hq, L, D]; the gate of row (b, l) is at g +
+// (b L + l) gs: Hq values (per head) or Hq x D (per dim).
 __global__ __launch_bounds__(256) void gate_heads_kernel(const uint16_t* __restrict__ attn,
-                                                         const uint16_t* __restrict__ g,
+                                                         const uint16_t* __restrict__ g, int64_t gs,
                                                          uint16_t* __restrict__ out, int64_t B,
                                                          int Hq, int64_t L, int per_dim) {
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -65,10 +97,11 @@ __global__ __launch_bounds__(256) void gate_heads_kernel(const uint16_t* __restr
   const int h = (int)(bh % Hq);
   const int64_t b = bh / Hq;
   const uint4 a = reinterpret_cast<const uint4*>(attn + rowi * ND)[c];
-  const int64_t orow = (b * L + l) * Hq + h;  // row of out [B, L, Hq, D] and of a per-dim gate
+  const int64_t orow = (b * L + l) * Hq + h;  // row of out [B, L, Hq, D]
+  const uint16_t* gr = g + (b * L + l) * gs;
   uint32_t aw[4] = {a.x, a.y, a.z, a.w}, ow[4];
   if (per_dim) {
-    const uint4 gv = reinterpret_cast<const uint4*>(g + orow * ND)[c];
+    const uint4 gv = reinterpret_cast<const uint4*>(gr + h * ND)[c];
     const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -78,7 +111,7 @@ __global__ __launch_bounds__(256) void gate_heads_kernel(const uint16_t* __restr
               ((uint32_t)f32_to_bf16(bf16_hi(aw[j]) * g1) << 16);
     }
   } else {
-    const float gate = bf16_to_f32(f32_to_bf16(softplus_f(bf16_to_f32(g[orow]))));
+    const float gate = bf16_to_f32(f32_to_bf16(softplus_f(bf16_to_f32(gr[h]))));
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       ow[j] = (uint32_t)f32_to_bf16(bf16_lo(aw[j]) * gate) |
@@ -538,18 +571,65 @@ extern "C" int lq_qk_norm_rope(const uint16_t* q, const uint16_t* k, uint16_t* q
   return LQ_OK;
 }
 
-extern "C" int lq_gate_heads(const uint16_t* attn, const uint16_t* gate, uint16_t* out, int64_t B,
-                             int64_t Hq, int64_t L, int64_t D, int per_dim, void* stream) {
-  using namespace lq;
-  clear_error();
+namespace lq {
+namespace {
+int gate_heads(const uint16_t* attn, const uint16_t* gate, int64_t gate_stride, uint16_t* out,
+               int64_t B, int64_t Hq, int64_t L, int64_t D, int per_dim, hipStream_t st) {
   LQ_CHECK_ARG(D == ND, "head_dim must be 128 (got %lld)", (long long)D);
   LQ_CHECK_ARG(B >= 1 && Hq >= 1 && L >= 1, "bad shape");
   LQ_CHECK_ARG(attn && gate && out && attn != out, "null or aliased pointer");
+  LQ_CHECK_ARG(gate_stride >= (per_dim ? Hq * D : Hq) &&
+                   (!per_dim || (gate_stride % 8 == 0 && ((uintptr_t)gate & 15) == 0)),
+               "a per-dim gate needs 16-byte aligned rows of at least Hq x 128 (stride %lld)",
+               (long long)gate_stride);
   const int64_t total = B * Hq * L * (ND / 8);
   LQ_CHECK_ARG(total / 256 < (int64_t)INT32_MAX, "too many rows");
-  hipStream_t st = (hipStream_t)stream;
   gate_heads_kernel<<<dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st>>>(
-      attn, gate, out, B, (int)Hq, L, per_dim ? 1 : 0);
+      attn, gate, gate_stride, out, B, (int)Hq, L, per_dim ? 1 : 0);
   LQ_CHECK_LAUNCH("gate_heads_kernel");
+  return LQ_OK;
+}
+}  // namespace
+}  // namespace lq
+
+extern "C" int lq_gate_heads(const uint16_t* attn, const uint16_t* gate, uint16_t* out, int64_t B,
+                             int64_t Hq, int64_t L, int64_t D, int per_dim, void* stream) {
+  lq::clear_error();
+  return lq::gate_heads(attn, gate, per_dim ? Hq * D : Hq, out, B, Hq, L, D, per_dim,
+                        (hipStream_t)stream);
+}
+
+extern "C" int lq_gate_heads_strided(const uint16_t* attn, const uint16_t* gate,
+                                     int64_t gate_stride, uint16_t* out, int64_t B, int64_t Hq,
+                                     int64_t L, int64_t D, int per_dim, void* stream) {
+  lq::clear_error();
+  return lq::gate_heads(attn, gate, gate_stride, out, B, Hq, L, D, per_dim, (hipStream_t)stream);
+}
+
+extern "C" int lq_qkv_norm_rope(const uint16_t* proj, int64_t N, uint16_t* q_out, uint16_t* k_out,
+                                uint16_t* v_out, const uint16_t* q_norm_w,
+                                const uint16_t* k_norm_w, int64_t B, int64_t Hq, int64_t Hkv,
+                                int64_t L, int64_t D, float eps, const float* inv_freq,
+                                int64_t rot_dims, float mscale, int64_t offset, void* stream) {
+  using namespace lq;
+  clear_error();
+  LQ_CHECK_ARG(D == ND, "head_dim must be 128 (got %lld)", (long long)D);
+  LQ_CHECK_ARG(B >= 1 && Hq >= 1 && Hkv >= 1 && L >= 1 && Hq <= 1024 && Hkv <= 1024,
+               "bad shape B=%lld Hq=%lld Hkv=%lld L=%lld", (long long)B, (long long)Hq,
+               (long long)Hkv, (long long)L);
+  LQ_CHECK_ARG(N >= (Hq + 2 * Hkv) * D, "rows of %lld values are shorter than the heads",
+               (long long)N);
+  LQ_CHECK_ARG(rot_dims >= 0 && rot_dims <= D && rot_dims % 4 == 0,
+               "rot_dims must be a multiple of 4 in [0, 128] (got %lld)", (long long)rot_dims);
+  LQ_CHECK_ARG(offset >= 0, "negative offset");
+  LQ_CHECK_ARG(proj && q_out && k_out && v_out && q_norm_w && k_norm_w &&
+                   (inv_freq || rot_dims == 0),
+               "null pointer");
+  const int64_t items = B * L * (Hq + 2 * Hkv);
+  LQ_CHECK_ARG(items / 4 < (int64_t)INT32_MAX, "too many rows");
+  qkv_norm_rope_kernel<<<dim3((unsigned)((items + 3) / 4)), dim3(256), 0, (hipStream_t)stream>>>(
+      proj, N, q_out, k_out, v_out, q_norm_w, k_norm_w, B * L, (int)Hq, (int)Hkv, L, eps, inv_freq,
+      (int)rot_dims, mscale, offset);
+  LQ_CHECK_LAUNCH("qkv_norm_rope_kernel");
   return LQ_OK;
 }

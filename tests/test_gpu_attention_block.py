@@ -485,3 +485,38 @@ def test_attention_block_quantized_decode_routes_packed_kv(dev, bits):
         assert err <= 2e-2 * scale, (L, err, scale)
         if L > 1:
             assert torch.equal(a, want)  # multi-row steps take the dequantize path in both
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,gate", [(1, 32, 8, 8, 32), (2, 3, 1, 5, 3), (1, 6, 2, 17, 6 * 128),
+                                             (1, 4, 4, 1, 4)])
+def test_qkv_norm_rope_and_strided_gate_equal_the_separate_ops(dev, B, Hq, Hkv, L, gate):
+    """The projection taken apart in one launch, and the gate read from its columns (an odd row
+    length, a per-dim gate): bit for bit the copies followed by lq_qk_norm_rope and lq_gate_heads."""
+    from lagunalab_amd import _lib
+    lib = _lib.load()
+    sp = _lib.stream_ptr(dev)
+    g = torch.Generator(device="cpu").manual_seed(L + Hq)
+    rnd = lambda *s: torch.randn(s, generator=g).to(torch.bfloat16).to(dev)  # noqa: E731
+    N, D = (Hq + 2 * Hkv) * 128 + gate, 128
+    proj, qw, kw, attn = rnd(B, L, N), rnd(D), rnd(D), rnd(B, Hq, L, D)
+    inv = (5e5 ** (-torch.arange(32) / 32)).to(dev)
+    parts = torch.split(proj, [Hq * D, Hkv * D, Hkv * D, gate], dim=-1)
+    q, k, v = (p.reshape(B, L, -1, D).transpose(1, 2).clone(memory_format=torch.contiguous_format)
+               for p in parts[:3])
+    _lib.check(lib.lq_qk_norm_rope(q.data_ptr(), k.data_ptr(), q.data_ptr(), k.data_ptr(),
+                                   qw.data_ptr(), kw.data_ptr(), B, Hq, Hkv, L, D, 1e-6,
+                                   inv.data_ptr(), 64, 1.0, 77, None, sp), "lq_qk_norm_rope")
+    q2, k2, v2 = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    _lib.check(lib.lq_qkv_norm_rope(proj.data_ptr(), N, q2.data_ptr(), k2.data_ptr(), v2.data_ptr(),
+                                    qw.data_ptr(), kw.data_ptr(), B, Hq, Hkv, L, D, 1e-6,
+                                    inv.data_ptr(), 64, 1.0, 77, sp), "lq_qkv_norm_rope")
+    assert torch.equal(q, q2) and torch.equal(k, k2) and torch.equal(v, v2)
+    y = torch.empty((B, L, Hq, D), dtype=torch.bfloat16, device=dev)
+    y2 = torch.empty_like(y)
+    per_dim = int(gate != Hq)
+    gc = parts[3].contiguous()
+    _lib.check(lib.lq_gate_heads(attn.data_ptr(), gc.data_ptr(), y.data_ptr(), B, Hq, L, D, per_dim,
+                                 sp), "lq_gate_heads")
+    _lib.check(lib.lq_gate_heads_strided(attn.data_ptr(), parts[3].data_ptr(), N, y2.data_ptr(), B, Hq,
+                                         L, D, per_dim, sp), "lq_gate_heads_strided")
+    assert torch.equal(y, y2)
