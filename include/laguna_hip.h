@@ -282,6 +282,11 @@ int lq_add_rms_norm(const uint16_t* h, const uint16_t* d, const uint16_t* w, uin
 int lq_gemv_bf16(const uint16_t* W, const uint16_t* x, uint16_t* y, int64_t N, int64_t K,
                  void* stream);
 
+/* y = x W^T for up to 16 rows: W bf16 [N, K], x bf16 [M, K], y bf16 [M, N]; fp32 accumulation; K a
+ * multiple of 8; W and x 16-byte aligned. */
+int lq_gemm_rows_bf16(const uint16_t* W, const uint16_t* x, uint16_t* y, int64_t M, int64_t N,
+                      int64_t K, void* stream);
+
 /*
  * The projections of a decode step with their neighbours fused in (one input row, W bf16 [N, K],
  * K a multiple of 8 up to 4096):

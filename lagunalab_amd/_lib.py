@@ -52,6 +52,7 @@ SIGNATURES = {
     "lq_gate_heads_strided": (i32, [vp, vp, i64, vp, i64, i64, i64, i64, i32, vp]),
     "lq_gate_heads": (i32, [vp, vp, vp, i64, i64, i64, i64, i32, vp]),
     "lq_add_rms_norm": (i32, [vp, vp, vp, vp, vp, i64, i64, f32, vp]),
+    "lq_gemm_rows_bf16": (i32, [vp, vp, vp, i64, i64, i64, vp]),
     "lq_gemv_bf16": (i32, [vp, vp, vp, i64, i64, vp]),
     "lq_gemv_fused": (i32, [vp, vp, vp, vp, vp, i64, i64, i32, f32, i32, vp]),
     "lq_q8_decode_norm_append_attn": (i32, [vp, vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64,

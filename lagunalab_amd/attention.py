@@ -8,8 +8,8 @@ mlx-lm's SDPA routes it), SDPA over the returned K/V otherwise, then the softplu
 ``o_proj``. The pieces:
 
 * one GEMM for q, k, v and the gate logits (the four projection weights concatenated), one for
-  ``o_proj``: ``lq_gemv_bf16`` for a single row (a decode step), hipBLASLt through torch for
-  more rows;
+  ``o_proj``: ``lq_gemv_bf16`` for a single row (a decode step), ``lq_gemm_rows_bf16`` for up to
+  16 (a verify block), hipBLASLt through torch for more;
 * ``lq_qkv_norm_rope``: the projection taken apart, the q and k RMSNorms and the rotary embedding
   of both in one launch
   (frequencies from :func:`rope_frequencies`: mlx-lm's default or YaRN RoPE, partial rotary);
@@ -89,16 +89,29 @@ def _sdpa(q, k, v, mask, scale):
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x @ w.T`` for bf16 ``x [..., K]`` and ``w [N, K]``: one row (a decode step) runs
-    ``lq_gemv_bf16`` (weight-streaming, HBM-bound), more rows the library GEMM."""
+    ``lq_gemv_bf16`` (weight-streaming, HBM-bound), 2 to 16 rows (a verify block) the matrix-core
+    form of it, ``lq_gemm_rows_bf16``, more rows the library GEMM. Every workgroup of the row form
+    reads all of x, so long rows go to the library where that costs more than its tiling: us per
+    call, row form / library, 2,048 outputs: 16 x 4,096 9.4 / 11.6, 8 x 6,144 11.8 / 11.7, 16 x
+    6,144 13.9 / 11.5; 6,176 outputs of 2,048: 2 rows 7.8 / 12.6, 8 9.4 / 12.9, 16 11.1 / 12.7."""
     K = x.shape[-1]
-    if x.numel() != K:
+    rows = x.numel() // K if K else 0
+    if rows != 1 and not (
+            2 <= rows <= 16 and K <= (4096 if rows > 8 else 6144) and K % 8 == 0 and w.dim() == 2 and w.shape[1] == K and w.shape[0]
+            and x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and w.is_contiguous()
+            and x.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
         return torch.matmul(x, w.t())
     lib = _lib.load()
     dev = _lib.require_device(x, w)
     x = x.contiguous()
     y = torch.empty((*x.shape[:-1], w.shape[0]), dtype=torch.bfloat16, device=dev)
-    _lib.check(lib.lq_gemv_bf16(w.data_ptr(), x.data_ptr(), y.data_ptr(), w.shape[0], K,
-                                _lib.stream_ptr(dev)), "lq_gemv_bf16")
+    if rows == 1:
+        _lib.check(lib.lq_gemv_bf16(w.data_ptr(), x.data_ptr(), y.data_ptr(), w.shape[0], K,
+                                    _lib.stream_ptr(dev)), "lq_gemv_bf16")
+    else:
+        _lib.check(lib.lq_gemm_rows_bf16(w.data_ptr(), x.data_ptr(), y.data_ptr(), rows, w.shape[0],
+                                         K, _lib.stream_ptr(dev)), "lq_gemm_rows_bf16")
     return y
 
 

@@ -503,6 +503,79 @@ extern "C" int lq_gemv_norm_rope(const uint16_t* W, const uint16_t* x, const uin
 }
 
 
+namespace lq {
+namespace {
+
+typedef __bf16 bfrag_t __attribute__((ext_vector_type(8)));
+typedef float facc_t __attribute__((ext_vector_type(4)));
+
+// y [M, N] = x [M, K] W^T for M <= 16 rows (the projections of a verify block): weight streaming
+// with matrix cores. A workgroup of 8 waves takes 16 outputs of every row, each wave an eighth of K
+// (one 16x16x32 MFMA per 32 of it: A = 16 weight rows, B = the rows of x, rows past M repeating
+// the last), 8 steps' loads in flight; the waves' fp32 sums meet in LDS. Bound by the weights'
+// stream and its ramp (25 and 17 MB, 3-5 us at a large copy's rate) and by the rows of x that
+// every workgroup reads: 8 rows, 6,176 x 2,048 in 9.4 us and 2,048 x 4,096 in 8.1, where the
+// library takes 12.9 and 11.6 (in a graph, weights not cached).
+constexpr int GW = 8;
+__global__ __launch_bounds__(64 * GW) void gemm_rows_kernel(const uint16_t* __restrict__ W,
+                                                            const uint16_t* __restrict__ x,
+                                                            uint16_t* __restrict__ y, int M,
+                                                            int64_t N, int K) {
+  __shared__ facc_t red[GW][64];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int lc = lane & 15, kq = lane >> 4;
+  const int64_t n0 = (int64_t)blockIdx.x * 16;
+  const uint16_t* wr = W + min(n0 + lc, N - 1) * K;
+  const uint16_t* xr = x + (int64_t)min(lc, M - 1) * K;
+  const int kw = (K + 32 * GW - 1) / (32 * GW) * 32;
+  const int k0 = wv * kw, k1 = min(K, k0 + kw);
+  facc_t acc = {0.f, 0.f, 0.f, 0.f};
+  for (int k = k0; k < k1; k += 256) {
+    uint4 a[8], b[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {  // K is a multiple of 8: a chunk lies inside or past the end
+      const int kc = min(k + 32 * s + 8 * kq, K - 8);
+      a[s] = *reinterpret_cast<const uint4*>(wr + kc);
+      b[s] = *reinterpret_cast<const uint4*>(xr + kc);
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      if (k + 32 * s + 8 * kq >= k1) a[s] = b[s] = make_uint4(0u, 0u, 0u, 0u);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bfrag_t, a[s]),
+                                                    __builtin_bit_cast(bfrag_t, b[s]), acc, 0, 0, 0);
+    }
+  }
+  red[wv][lane] = acc;
+  __syncthreads();
+  if (wv != 0 || lc >= M) return;
+#pragma unroll
+  for (int w = 1; w < GW; ++w) acc += red[w][lane];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {  // acc[r]: output n0 + 4 kq + r of row lc
+    const int64_t n = n0 + 4 * kq + r;
+    if (n < N) y[(int64_t)lc * N + n] = f32_to_bf16(acc[r]);
+  }
+}
+
+}  // namespace
+}  // namespace lq
+
+extern "C" int lq_gemm_rows_bf16(const uint16_t* W, const uint16_t* x, uint16_t* y, int64_t M,
+                                 int64_t N, int64_t K, void* stream) {
+  using namespace lq;
+  clear_error();
+  LQ_CHECK_ARG(M >= 1 && M <= 16, "%lld rows outside [1, 16]", (long long)M);
+  LQ_CHECK_ARG(N >= 1 && N < (int64_t)1 << 31 && K >= 8 && K % 8 == 0 && K < (int64_t)1 << 24,
+               "bad shape N=%lld K=%lld (K a multiple of 8)", (long long)N, (long long)K);
+  LQ_CHECK_ARG(W && x && y, "null pointer");
+  LQ_CHECK_ARG((((uintptr_t)W | (uintptr_t)x) & 15) == 0, "W and x must be 16-byte aligned");
+  gemm_rows_kernel<<<dim3((unsigned)((N + 15) / 16)), dim3(64 * GW), 0, (hipStream_t)stream>>>(
+      W, x, y, (int)M, N, (int)K);
+  LQ_CHECK_LAUNCH("gemm_rows_kernel");
+  return LQ_OK;
+}
+
 extern "C" int lq_gemv_bf16(const uint16_t* W, const uint16_t* x, uint16_t* y, int64_t N,
                             int64_t K, void* stream) {
   using namespace lq;

@@ -520,3 +520,19 @@ def test_qkv_norm_rope_and_strided_gate_equal_the_separate_ops(dev, B, Hq, Hkv, 
     _lib.check(lib.lq_gate_heads_strided(attn.data_ptr(), parts[3].data_ptr(), N, y2.data_ptr(), B, Hq,
                                          L, D, per_dim, sp), "lq_gate_heads_strided")
     assert torch.equal(y, y2)
+
+
+@pytest.mark.parametrize("M,N,K", [(2, 16, 8), (16, 17, 264), (8, 6176, 2048), (5, 2048, 4096),
+                                   (3, 1, 40), (15, 100, 2056), (7, 48, 6144)])
+def test_gemm_rows(dev, M, N, K):
+    """The projections of 2 to 16 rows: outputs past a 16-column tile, K that leaves waves empty or
+    with part of a step. Against float64 on the same bf16 values: half a bf16 step of the result and
+    the fp32 sums' own error (K terms of 2^-24 of their absolute sum)."""
+    from lagunalab_amd.attention import linear
+    g = torch.Generator(device="cpu").manual_seed(M + N + K)
+    x = torch.randn((1, M, K), generator=g).to(torch.bfloat16)
+    w = (torch.randn((N, K), generator=g) * 0.05).to(torch.bfloat16)
+    got = linear(x.to(dev), w.to(dev)).double().cpu()
+    want = x.double() @ w.double().t()
+    bound = want.abs() * 2.0 ** -8 + (x.double().abs() @ w.double().abs().t()) * K * 2.0 ** -24
+    assert got.shape == (1, M, N) and bool(((got - want).abs() <= bound).all())
