@@ -23,6 +23,7 @@ from __future__ import annotations
 import math
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -87,6 +88,19 @@ def _sdpa(q, k, v, mask, scale):
     return torch.matmul(p, v.float()).reshape(B, Hq, Lq, D).to(q.dtype)
 
 
+def _row_form(x, w, rows, K):
+    """Whether ``lq_gemm_rows_bf16`` takes this product: what the kernel reads (bf16, contiguous,
+    16-byte aligned), and plain tensors outside autograd, forward-mode and function transforms,
+    which only the library product supports."""
+    return (K <= (4096 if rows > 8 else 6144) and K % 8 == 0
+            and w.dim() == 2 and w.shape[1] == K and w.shape[0] > 0
+            and x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device
+            and type(x) is type(w) is torch.Tensor
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+            and forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and x.is_contiguous() and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x @ w.T`` for bf16 ``x [..., K]`` and ``w [N, K]``: one row (a decode step) runs
     ``lq_gemv_bf16`` (weight-streaming, HBM-bound), 2 to 16 rows (a verify block) the matrix-core
@@ -96,11 +110,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     6,144 13.9 / 11.5; 6,176 outputs of 2,048: 2 rows 7.8 / 12.6, 8 9.4 / 12.9, 16 11.1 / 12.7."""
     K = x.shape[-1]
     rows = x.numel() // K if K else 0
-    if rows != 1 and not (
-            2 <= rows <= 16 and K <= (4096 if rows > 8 else 6144) and K % 8 == 0 and w.dim() == 2 and w.shape[1] == K and w.shape[0]
-            and x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and w.is_contiguous()
-            and x.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0
-            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
+    if rows != 1 and not (2 <= rows <= 16 and _row_form(x, w, rows, K)):
         return torch.matmul(x, w.t())
     lib = _lib.load()
     dev = _lib.require_device(x, w)

@@ -47,3 +47,23 @@ def test_yarn_limits_and_mscale():
 def test_unknown_rope_type_rejected():
     with pytest.raises(ValueError, match="rope_type"):
         rope_frequencies(128, {"rope_type": "llama3", "rope_theta": 1e4})
+
+
+def test_row_form_leaves_transforms_and_other_layouts_to_the_library():
+    """linear() of 2 to 16 rows: off the GPU, under vmap or forward mode, with gradients wanted, in
+    another type or layout, the library product is what runs."""
+    import torch
+    from torch.autograd import forward_ad
+    from lagunalab_amd.attention import linear
+    g = torch.Generator().manual_seed(1)
+    x, w = torch.randn((4, 64), generator=g), torch.randn((24, 64), generator=g)
+    want = x @ w.t()
+    assert torch.equal(linear(x, w), want)
+    assert torch.allclose(torch.vmap(lambda a: linear(a, w))(x.reshape(2, 2, 64)).reshape(4, 24), want)
+    xg = x.clone().requires_grad_()
+    linear(xg, w).sum().backward()
+    assert torch.allclose(xg.grad, w.sum(0).expand(4, 64), atol=1e-4)
+    with forward_ad.dual_level():
+        d = linear(forward_ad.make_dual(x, torch.ones_like(x)), w)
+        assert torch.allclose(forward_ad.unpack_dual(d).tangent, w.sum(1).expand(4, 24), atol=1e-4)
+    assert torch.equal(linear(x, w.t().contiguous().t()), x @ w.t().contiguous())
