@@ -34,9 +34,11 @@
 //   4t+3    dequantize K(t+1)        P.V(t)
 //
 // K(t+1) overwrites K(t) after both halves' Q.K^T(t), V(t) overwrites V(t-1) after both halves'
-// P.V(t-1), so one fp16 K and one V^T buffer suffice. Raw tile t+2 is issued in slot 4t+1 (its
-// slot held raw t, whose K was dequantized in slot 4t-1 and V in slot 4t) and waited for two
-// tiles later.
+// P.V(t-1), so one fp16 K and one V^T buffer suffice. The codes of raw tile t+2 and the words of
+// t+3 go into t's slots once both dequantizations of t are done, from each half's softmax slot, and
+// are waited for a tile later. Vector phases run at a raised wave priority: their instructions set
+// the pace and the matrix phases' issue only every 16 cycles (2,048 rows at 82,671 keys: 2,437 ->
+// 2,407 us against 2,429 and 2,414 of an unchanged kernel beside them).
 // Tiles past a wave's last row are skipped by that wave (it keeps its copy and dequantization
 // duties); tiles straddling its rows' bounds are masked per row. Rows past the chunk (a ragged last
 // block) read no q and store nothing. Keys past n-1 are never read: copies clamp their rows to n-1.
@@ -232,6 +234,7 @@ __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
   // (the thread index is re-read through an empty asm in each call, so that the compiler
   // recomputes these addresses in the slot instead of holding them in registers across the loop)
   auto dequant_k = [&](const PrefillRaw& rw, const PrefillWords& wd, int kk) {
+    __builtin_amdgcn_s_setprio(2);
     int tr = ta;
     asm volatile("" : "+v"(tr));
     const int dc = tr & 7;  // 16 codes of key (tr >> 3) + 32 i, dims 16 dc .. 16 dc + 15
@@ -277,6 +280,7 @@ __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
   // (source lane s addresses key T[s / 2], bytes 8 (s % 2) of the window; the raw V rows are
   // stored swizzled by 16-byte chunk, see the copies).
   auto dequant_v = [&](const PrefillRaw& rw, const PrefillWords& wd, int kv) {
+    __builtin_amdgcn_s_setprio(2);
     int ln = lane;
     asm volatile("" : "+v"(ln));
     const int e = wv - PW / 2, qg = ln >> 4, i = ln & 15;
@@ -452,6 +456,7 @@ __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
   // maxima (0 before the first): the accumulators start at -mref
   int kq = 0;  // the factor 2^kq that qb holds
   auto qk = [&]() {
+    __builtin_amdgcn_s_setprio(0);
     if (RANGE && kk != kq) {  // wave-uniform, rare: this tile's K has another factor
       kq = kk;
       int ln = lane;
@@ -490,6 +495,7 @@ __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
   };
   // softmax per N tile: masking, lazy rescale, P in fp16 (its row sums are taken by P.V)
   auto softmax = [&](int t0, bool full) {
+    __builtin_amdgcn_s_setprio(2);
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
       if (!full) {
@@ -540,6 +546,7 @@ __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
   // out^T[16 dt + 4 lq4 + r][row 16 nt + lc] += V^T[dims][slots] P^T[slots][rows]
   int kv_acc = 0;  // the factor 2^-kv_acc that the accumulators hold
   auto pv = [&](int snext) {  // ends with the factors of the next tile (its range in sm.rng[snext])
+    __builtin_amdgcn_s_setprio(0);
     kv_acc = kv;
     uint4 rnext;
     if (RANGE) rnext = *reinterpret_cast<const uint4*>(sm.rng[snext]);
