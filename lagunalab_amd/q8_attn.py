@@ -374,8 +374,9 @@ def q8_prefill_attention(q, keys, values, n, scale):
 
     q [B, Hq, L, 128] for the chunk's positions n-L .. n-1, whose K/V are already the last L of
     the first ``n`` cache rows; row i sees keys 0 .. n-L+i. Any L >= 1. Chunks of more than 16
-    rows run the prefill kernel (256 query rows per workgroup over shared, once-dequantized K/V
-    tiles), up to 16 the verify kernel. Returns [B, Hq, L, 128] in q's dtype."""
+    rows run the prefill kernel (256 query rows per workgroup over shared K/V tiles: dequantized to
+    fp16 for 1, 2, 4 and 8 query heads per KV head, the exact codes for other groupings), up to 16
+    the verify kernel. Returns [B, Hq, L, 128] in q's dtype."""
     B, Hq, L, D = q.shape
     kc, ks, kb = keys
     Hkv = kc.shape[1]

@@ -113,9 +113,10 @@ def test_v_scales_changing_across_the_cache(dev, B):
 
 
 # ------------------------------------------------------------------------------------- prefill
-# For groupings other than 1, 2, 4 and 8 the prefill kernel takes q, K and V in fp16 with
-# power-of-two factors per tile; the float64 oracle bounds it by the operands' 2^-11 steps: a score of size s moves by about s 2^-11 (peaked
-# scores are why the wide-q cases use fewer, smaller keys), P and V by 2^-11 relative each.
+# For groupings other than 1, 2, 4 and 8 the prefill kernel keeps the verify kernel's arithmetic: exact
+# codes as operands, the affine terms in 32 bits, P times the V scale in fp16 (2^-11 relative) with a
+# power-of-two factor per quant group and 64-key tile. The bars of the next two tests, from the operands'
+# 2^-11 steps (a score of size s moving by s 2^-11), leave it room.
 
 @pytest.mark.parametrize("G", [6, 3])
 @pytest.mark.parametrize("qstd,kstd,vstd", [(1e-4, 1.0, 1.0), (1.0, 1.0, 1e-6), (1.0, 1.0, 1e5),
@@ -147,9 +148,9 @@ def test_prefill_operand_range(dev, G, qstd, kstd, vstd):
 @pytest.mark.parametrize("G", [6, 3])
 def test_prefill_factors_change_between_tiles(dev, G):
     """K and V whose sizes jump by powers of two between 300-row regions (so that tiles straddle
-    them): the V factor rises and falls, K's factor moves q's. The keys of the smallest-V region
-    get the largest scores. (V sizes 2^-20 apart at most: where a tile straddles the regions, the
-    small values stay normal fp16 numbers below a largest one of 2^12 to 2^15.)"""
+    them): the V factor rises and falls. The keys of the smallest-V region get the largest scores.
+    (V sizes 2^-20 apart: where a tile straddles the regions, P times the small V scales is 2^-16 or
+    less of fp16's range, steps of 2^-9 of its largest value.)"""
     from lagunalab_amd.q8_attn import q8_prefill_attention
     from lagunalab_amd.quant import quantize_into
     rng = np.random.default_rng(78)
@@ -178,3 +179,101 @@ def test_prefill_factors_change_between_tiles(dev, G):
     mag = np.abs(want).max(-1, keepdims=True)
     err = np.abs(got.float().cpu().numpy() - want)
     assert np.all(err <= 8e-3 * mag + RTOL * np.abs(want)), float((err / mag).max())
+
+
+def _buffers(dev, x, cap):
+    """x [1, H, n, 128] quantized into full-capacity 8-bit buffers."""
+    from lagunalab_amd.quant import quantize_into
+    H = x.shape[1]
+    c = (torch.zeros((1, H, cap, 128), dtype=torch.uint8, device=dev),
+         torch.zeros((1, H, cap, 2), dtype=torch.bfloat16, device=dev),
+         torch.zeros((1, H, cap, 2), dtype=torch.bfloat16, device=dev))
+    quantize_into(to_dev_bf16(Q.round_bf16(x), dev), *c, 0, 64, 8)
+    return c
+
+
+def _split(n, L, G, Hkv):
+    from lagunalab_amd import _lib
+    return _lib.load().lq_prefill_workspace_bytes(1, Hkv * G, Hkv, L, n) > 0
+
+
+@pytest.mark.parametrize("G,n,L,Hkv", [(6, 1000, 100, 2), (6, 8193, 256, 2), (3, 3000, 200, 2),
+                                       (12, 3000, 100, 1)])
+def test_prefill_of_other_groupings_is_as_exact_as_the_verify_kernel(dev, G, n, L, Hkv):
+    """Both take the exact codes as operands and the affine terms in 32 bits: the relative error
+    against 64 bits is the verify kernel's. It is a norm over 150,000 to 400,000 outputs, most of it
+    their bf16 rounding, so two draws of it agree to about 0.5 / sqrt(150,000) = 0.13%; K and V
+    rounded to fp16 before the products show 3 to 5%. Scores with a standard deviation of 2."""
+    from lagunalab_amd.q8_attn import _prefill_blocked, q8_prefill_attention
+    rng = np.random.default_rng(G + n)
+    kq, vq = (_buffers(dev, Q.randn_bf16(rng, (1, Hkv, n, 128)), n + 3) for _ in range(2))
+    q = Q.round_bf16(2 * Q.randn_bf16(rng, (1, Hkv * G, L, 128)))
+    qd = to_dev_bf16(q, dev)
+    want = A.fused_attention(q, cache_np(kq), cache_np(vq), n, 128 ** -0.5, causal=True)
+
+    def error(out):
+        return np.linalg.norm(out.float().cpu().numpy() - want) / np.linalg.norm(want)
+    got = error(q8_prefill_attention(qd, kq, vq, n, 128 ** -0.5))
+    verify = error(_prefill_blocked(qd, kq, vq, n, 128 ** -0.5))
+    assert got <= 1.01 * verify, (got, verify)
+
+
+@pytest.mark.parametrize("G", [6, 3])
+@pytest.mark.parametrize("n,L", [(1000, 70), (3000, 70)], ids=["whole", "split"])
+@pytest.mark.parametrize("kind", ["far keys", "large scores", "V groups", "V tiles"])
+def test_prefill_operands_far_apart(dev, kind, n, L, G):
+    """What the verify kernel serves and a dequantized fp16 operand does not hold: keys 2^36 times
+    others of their tile (with scores far below theirs), scores of 2^30 and more, V groups of one
+    head 2^-18 of each other, V sizes that jump by powers of two between regions of five 64-key tiles
+    (at 1,000 keys in whole blocks: the exponent changes within one walk of the keys)."""
+    from lagunalab_amd.q8_attn import q8_prefill_attention
+    Hkv, cap = 2, n + 40
+    assert _split(n, L, G, Hkv) == (n == 3000)
+    rng = np.random.default_rng(n + G)
+    q = Q.randn_bf16(rng, (1, Hkv, 1, 1, 128)) * np.float32(4.0)
+    q = Q.round_bf16(q + 0.3 * Q.randn_bf16(rng, (1, Hkv, G, L, 128))).reshape(1, Hkv * G, L, 128)
+    qdir = q[0, ::G, 0] / np.linalg.norm(q[0, ::G, 0], axis=-1, keepdims=True)
+    k, v = (Q.randn_bf16(rng, (1, Hkv, n, 128)) for _ in range(2))
+    if kind == "far keys":
+        k[:, :, ::2] -= np.float32(2.0 ** 36) * qdir[None, :, None, :]
+    elif kind == "large scores":
+        k *= np.float32(2.0 ** 16)
+        q = Q.round_bf16(Q.randn_bf16(rng, q.shape) * np.float32(2.0 ** 16))
+    elif kind == "V groups":
+        v[..., 64:] *= np.float32(2.0 ** -18)
+    else:
+        region = (np.arange(n) // 320) % 3
+        k += np.where(region == 1, 6.0, -6.0).astype(np.float32)[:, None] * qdir[None, :, None, :]
+        v *= (np.float32(2.0) ** np.array([4, -14, -5])[region]).astype(np.float32)[:, None]
+    kq, vq = _buffers(dev, k, cap), _buffers(dev, v, cap)
+    got = q8_prefill_attention(to_dev_bf16(q, dev), kq, vq, n, 128 ** -0.5).float().cpu().numpy()
+    want = A.fused_attention(q, cache_np(kq), cache_np(vq), n, 128 ** -0.5, causal=True)
+    assert np.isfinite(got).all()
+    for g in (slice(0, 64), slice(64, 128)):
+        # the parity bar, against each row's own largest value of the group
+        mag = np.abs(want[..., g]).max(-1, keepdims=True)
+        err = np.abs(got[..., g] - want[..., g])
+        assert np.all(err <= 2e-3 * mag + RTOL * np.abs(want[..., g])), (kind, float((err / mag).max()))
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("word", ["K scale", "K bias", "V scale", "V bias"])
+def test_prefill_infinity_in_a_key_reaches_the_rows_that_see_it(dev, word, value):
+    """A NaN or infinity in one key of the chunk: the rows before it are what they are without it, the
+    rows from it on are not finite. (A K scale or bias of -inf times a q sum can also give a score of
+    -inf, a key without weight: rows with a NaN or a changed result both count as reached.)"""
+    from lagunalab_amd.q8_attn import q8_prefill_attention
+    rng = np.random.default_rng(9)
+    n, L, G, Hkv, at = 700, 90, 6, 1, 650  # the chunk begins at key 610
+    kq, vq = (_buffers(dev, Q.randn_bf16(rng, (1, Hkv, n, 128)), n) for _ in range(2))
+    q = to_dev_bf16(Q.randn_bf16(rng, (1, Hkv * G, L, 128)), dev)
+    clean = q8_prefill_attention(q, kq, vq, n, 128 ** -0.5).float()
+    buf = (kq if word[0] == "K" else vq)[1 if word.endswith("scale") else 2]
+    buf[0, 0, at, 0] = value
+    got = q8_prefill_attention(q, kq, vq, n, 128 ** -0.5).float()
+    i = at - (n - L)
+    assert torch.allclose(got[:, :, :i], clean[:, :, :i], rtol=2.0 ** -7, atol=0)
+    reached = ~torch.isclose(got[:, :, i:], clean[:, :, i:], rtol=2.0 ** -7, atol=0).all(-1)
+    assert bool(reached.all())
+    if value != value:
+        assert bool(got[:, :, i:].isnan().any(-1).all())
