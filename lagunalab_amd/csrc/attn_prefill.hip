@@ -958,9 +958,11 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(uint16_t* __restrict
       const int64_t r = row(j);
       const float2 ml = sp.part_ml[r];
       const f4_t o = *reinterpret_cast<const f4_t*>(sp.part_o + r * D + 4 * ln);
-      const float w = ml.y > 0.0f ? exp2_nonpos(ml.x - M) * ml.y : 0.0f;
-      if (w > 0.0f) acc += o * w;
-      den += w;
+      if (ml.y != 0.0f) {  // a part that saw keys; a NaN sum goes into the row's
+        const float w = exp2_nonpos(ml.x - M) * ml.y;
+        acc += o * w;
+        den += w;
+      }
     }
   }
   sh_acc[tr][grp][ln] = acc;
@@ -975,11 +977,13 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(uint16_t* __restrict
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     const float2 ml = sh_ml[tr][g];
-    const float w = ml.y > 0.0f ? exp2_nonpos(ml.x - mx) : 0.0f;
-    if (w > 0.0f) acc += sh_acc[tr][g][ln] * w;
-    den += w * ml.y;
+    if (ml.y != 0.0f) {
+      const float w = exp2_nonpos(ml.x - mx);
+      acc += sh_acc[tr][g][ln] * w;
+      den += w * ml.y;
+    }
   }
-  const f4_t o = acc * (den > 0.0f ? 1.0f / den : 0.0f);
+  const f4_t o = acc * (den != 0.0f ? 1.0f / den : 0.0f);
   const int i = (int)fdiv_u((uint32_t)f, sp.g), head = f - i * G;
   const uint32_t lo = (uint32_t)f32_to_bf16(o[0]) | ((uint32_t)f32_to_bf16(o[1]) << 16);
   const uint32_t hi = (uint32_t)f32_to_bf16(o[2]) | ((uint32_t)f32_to_bf16(o[3]) << 16);

@@ -930,6 +930,40 @@ def test_prefill_split_over_the_keys(dev, n, L, G, Hkv, B):
     assert_attn_close(out, want, "split, workspace of NaN")
 
 
+@pytest.mark.parametrize("G", [4, 6])
+@pytest.mark.parametrize("what", ["query", "key", "both"])
+def test_prefill_split_passes_nan_and_infinity_on(dev, G, what):
+    """A NaN or infinite query row, or a key with a NaN scale (in one share of the keys), gives the rows
+    that hold or see it NaN in a split chunk as in whole blocks (G = 4: the entry that never splits) and
+    in the verify kernel's blocks, and leaves the others as they are without it."""
+    from lagunalab_amd import _lib, q8_attn
+    lib = _lib.load()
+    n, L, Hkv = 6000, 40, 2
+    assert lib.lq_prefill_workspace_bytes(1, Hkv * G, Hkv, L, n) > 0
+    rng = np.random.default_rng(G)
+    kq, vq = make_cache(rng, 1, Hkv, n, n, dev)
+    q = to_dev_bf16(Q.randn_bf16(rng, (1, Hkv * G, L, 128)), dev)
+    clean = q8_attn.q8_prefill_attention(q, kq, vq, n, 0.09)
+    lost = torch.zeros((1, Hkv * G, L), dtype=torch.bool, device=dev)
+    if what != "key":
+        q[0, 1, 7, 3] = float("nan")
+        q[0, 2, 9] = float("inf")
+        lost[0, 1, 7] = lost[0, 2, 9] = True
+    if what != "query":
+        kq[1][0, 1, 1234, 0] = float("nan")
+        lost[0, G:] = True  # every row of KV head 1
+    got = q8_attn.q8_prefill_attention(q, kq, vq, n, 0.09)
+    assert torch.equal(got.isnan().all(-1), lost) and torch.equal(got.isnan().any(-1), lost)
+    assert torch.equal(got[~lost], clean[~lost])
+    blocked = q8_attn._prefill_blocked(q, kq, vq, n, 0.09)
+    assert torch.equal(blocked.isnan().any(-1) & lost, lost)
+    if G == 4:
+        whole = torch.empty_like(q)
+        assert lib.lq_q8_prefill_attn(q.data_ptr(), *(t.data_ptr() for t in (*kq, *vq)), 1, Hkv * G, Hkv,
+                                      L, 128, n, n, 0.09, whole.data_ptr(), _lib.stream_ptr(dev)) == 0
+        assert torch.equal(whole.isnan().all(-1), lost)
+
+
 def test_prefill_split_shares_cover_several_blocks(dev):
     """25 blocks per KV head on 10 workgroups each: shares of two and a half blocks (the end of one,
     a whole one, the start of the next), against the entry that never splits."""
