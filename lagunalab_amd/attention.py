@@ -24,6 +24,7 @@ import math
 
 import torch
 from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 from . import _lib
 
@@ -88,17 +89,30 @@ def _sdpa(q, k, v, mask, scale):
     return torch.matmul(p, v.float()).reshape(B, Hq, Lq, D).to(q.dtype)
 
 
+def _unwatched(*tensors):
+    """Whether an operation on these may be launched past torch's dispatcher: plain tensors, and nothing
+    that records, rewrites or casts what the dispatcher sees -- autograd, forward mode, function
+    transforms (vmap, grad), jit and fx tracing, compilation, dispatch and function modes (other than a
+    default device's) and autocast. Those get the library product, which they can see."""
+    return (all(type(t) is torch.Tensor for t in tensors)
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+            and forward_ad._current_level < 0
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and not torch._C._is_tracing() and not torch.compiler.is_compiling()
+            and torch._C._len_torch_dispatch_stack() == 0
+            and all(type(torch._C._get_function_stack_at(i)) is DeviceContext
+                    for i in range(torch._C._len_torch_function_stack()))
+            and not torch.is_autocast_enabled(tensors[0].device.type))
+
+
 def _row_form(x, w, rows, K):
     """Whether ``lq_gemm_rows_bf16`` takes this product: what the kernel reads (bf16, contiguous,
-    16-byte aligned), and plain tensors outside autograd, forward-mode and function transforms,
-    which only the library product supports."""
+    16-byte aligned), in a call that nothing watches."""
     return (K <= (4096 if rows > 8 else 6144) and K % 8 == 0
             and w.dim() == 2 and w.shape[1] == K and w.shape[0] > 0
             and x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device
-            and type(x) is type(w) is torch.Tensor
-            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
-            and forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
-            and x.is_contiguous() and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+            and x.is_contiguous() and w.is_contiguous() and _unwatched(x, w)
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -67,3 +67,47 @@ def test_row_form_leaves_transforms_and_other_layouts_to_the_library():
         d = linear(forward_ad.make_dual(x, torch.ones_like(x)), w)
         assert torch.allclose(forward_ad.unpack_dual(d).tangent, w.sum(1).expand(4, 24), atol=1e-4)
     assert torch.equal(linear(x, w.t().contiguous().t()), x @ w.t().contiguous())
+
+
+def test_unwatched_calls_only_outside_tracing_modes_and_autocast():
+    """The row form's launch is not seen by the dispatcher, so every context that works on what the
+    dispatcher sees has to be told apart from a plain call."""
+    import torch
+    from torch.autograd import forward_ad
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+    from lagunalab_amd.attention import _unwatched
+    x, w = torch.randn((4, 8)), torch.randn((3, 8))
+    seen = []
+
+    def call(a, b=w):
+        seen.append(_unwatched(a, b))
+        return a @ b.t()
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, fn, types, args=(), kwargs=None):
+            return fn(*args, **(kwargs or {}))
+
+    call(x)
+    with torch.inference_mode():
+        call(x)
+    with torch.device("cpu"):
+        call(x)
+    assert seen == [True] * 3
+    seen.clear()
+    torch.jit.trace(call, (x,), check_trace=False)
+    make_fx(call)(x)
+    make_fx(call, tracing_mode="fake")(x, w)
+    with FlopCounterMode(display=False):
+        call(x)
+    with torch.autocast("cpu", dtype=torch.bfloat16):
+        call(x)
+    with Mode():
+        call(x)
+    torch.vmap(call)(x)
+    call(x.clone().requires_grad_())
+    call(torch.nn.Parameter(x))
+    with forward_ad.dual_level():
+        call(forward_ad.make_dual(x, x))
+    assert len(seen) >= 10 and not any(seen)

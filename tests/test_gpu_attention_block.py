@@ -536,3 +536,23 @@ def test_gemm_rows(dev, M, N, K):
     want = x.double() @ w.double().t()
     bound = want.abs() * 2.0 ** -8 + (x.double().abs() @ w.double().abs().t()) * K * 2.0 ** -24
     assert got.shape == (1, M, N) and bool(((got - want).abs() <= bound).all())
+
+
+def test_row_products_are_seen_by_tracing_modes_and_autocast(dev):
+    """linear() of 4 rows traced (jit and fx) and called on other inputs, under a FLOP counter and under
+    autocast: the product itself is recorded, counted and cast, as the library's is."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils.flop_counter import FlopCounterMode
+    from lagunalab_amd.attention import linear
+    g = torch.Generator(device="cpu").manual_seed(4)
+    w = torch.randn((256, 1024), generator=g).to(torch.bfloat16).to(dev)
+    x, x2 = (torch.randn((4, 1024), generator=g).to(torch.bfloat16).to(dev) for _ in range(2))
+    want = torch.matmul(x2, w.t())
+    traced = torch.jit.trace(lambda a: linear(a, w), (x,), check_trace=False)
+    assert torch.equal(traced(x2), want)
+    assert torch.equal(make_fx(lambda a: linear(a, w))(x)(x2), want)
+    with FlopCounterMode(display=False) as flops:
+        linear(x, w)
+    assert flops.get_total_flops() == 2 * 4 * 256 * 1024
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert linear(x, w).dtype == torch.float16
