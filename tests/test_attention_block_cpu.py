@@ -97,8 +97,8 @@ def test_unwatched_calls_only_outside_tracing_modes_and_autocast():
     assert seen == [True] * 3
     seen.clear()
     torch.jit.trace(call, (x,), check_trace=False)
-    make_fx(call)(x)
-    make_fx(call, tracing_mode="fake")(x, w)
+    make_fx(lambda a, b: call(a, b))(x, w)
+    make_fx(lambda a, b: call(a, b), tracing_mode="fake")(x, w)
     with FlopCounterMode(display=False):
         call(x)
     with torch.autocast("cpu", dtype=torch.bfloat16):
