@@ -261,8 +261,8 @@ class DequantKVCache:
 
     def attend(self, queries, scale):
         """Attention straight off the packed cache: the fused decode kernel for one query row,
-        the fused causal verify kernel for a block of up to 16 rows, the blocked causal kernel
-        for longer chunks; the step's pending new rows are appended by the same call."""
+        the fused causal verify kernel for a block of up to 16 rows, the prefill kernel for
+        longer chunks; the step's pending new rows are appended by the same call. They stay pending if it raises, so the cache never holds rows that were not written."""
         from .q8_attn import (decode_append_attention, q8_decode_attention,
                               q8_prefill_attention, q8_verify_append_attention,
                               q8_verify_attention)
@@ -272,13 +272,14 @@ class DequantKVCache:
             k, v, row = self._pending
             if queries.shape[3] != 128:
                 raise AssertionError("head_dim 128")
-            self._pending = None
             if L == 1:
                 out = decode_append_attention(queries.to(torch.bfloat16), k, v, self.q.keys,
-                                              self.q.values, n=row, scale=scale)
-                return out.to(queries.dtype)
-            return q8_verify_append_attention(queries, k, v, self.q.keys, self.q.values, row,
-                                              scale)
+                                              self.q.values, n=row, scale=scale).to(queries.dtype)
+            else:
+                out = q8_verify_append_attention(queries, k, v, self.q.keys, self.q.values, row,
+                                                 scale)
+            self._pending = None
+            return out
         self._flush()
         if L == 1:
             return q8_decode_attention(queries, self.q.keys, self.q.values, self.q.offset, scale)

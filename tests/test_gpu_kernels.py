@@ -1005,3 +1005,20 @@ def test_dequantize_kv_bit_exact(dev, bits, gs, D, n, cap, B, H):
                 + b.float().repeat_interleave(gs, -1)).to(torch.bfloat16)
         assert torch.equal(got, want)
         assert torch.equal(dequantize(*buf, gs, bits, n=n), want)
+
+
+@pytest.mark.parametrize("L", [1, 3])
+def test_rows_stay_pending_when_attend_raises(dev, L):
+    """attend() refusing its queries (7 heads over 2 KV heads) leaves the step's rows pending: the next
+    read of the cache writes them."""
+    from lagunalab_amd.cache import DequantKVCache, QuantizedKVCache
+    rng = np.random.default_rng(L)
+    k, v = (to_dev_bf16(Q.randn_bf16(rng, (1, 2, 40 + L, 128)), dev) for _ in range(2))
+    cache, plain = DequantKVCache(fused_decode=True), QuantizedKVCache()
+    for c in (cache, plain):
+        c.update_and_fetch(k[:, :, :40], v[:, :, :40])
+        c.update_and_fetch(k[:, :, 40:], v[:, :, 40:])
+    with pytest.raises(ValueError):
+        cache.attend(torch.zeros((1, 7, L, 128), dtype=torch.bfloat16, device=dev), 0.09)
+    for a, b in zip(cache.state[0] + cache.state[1], plain.state[0] + plain.state[1]):
+        assert torch.equal(a, b)
