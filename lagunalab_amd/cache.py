@@ -261,14 +261,17 @@ class DequantKVCache:
 
     def attend(self, queries, scale):
         """Attention straight off the packed cache: the fused decode kernel for one query row,
-        the fused causal verify kernel for a block of up to 16 rows, the prefill kernel for
-        longer chunks; the step's pending new rows are appended by the same call. They stay pending if it raises, so the cache never holds rows that were not written."""
+        the fused causal verify kernel for a block of up to 16 rows and 64 query rows per KV head,
+        the prefill kernel for longer ones; the step's pending new rows are appended by the same
+        call. They stay pending if it raises, so the cache never holds rows that were not written."""
         from .q8_attn import (decode_append_attention, q8_decode_attention,
                               q8_prefill_attention, q8_verify_append_attention,
                               q8_verify_attention)
 
         L = queries.shape[2]
-        if self._pending is not None and self._pending[0].shape[2] == L:
+        # beyond a verify block's rows: the prefill kernel, on rows appended first
+        chunk = L > 16 or (L > 1 and queries.shape[1] * L > 64 * self.q.keys[0].shape[1])
+        if self._pending is not None and self._pending[0].shape[2] == L and not chunk:
             k, v, row = self._pending
             if queries.shape[3] != 128:
                 raise AssertionError("head_dim 128")
@@ -283,7 +286,7 @@ class DequantKVCache:
         self._flush()
         if L == 1:
             return q8_decode_attention(queries, self.q.keys, self.q.values, self.q.offset, scale)
-        if L > 16:
+        if chunk:
             return q8_prefill_attention(queries, self.q.keys, self.q.values, self.q.offset, scale)
         return q8_verify_attention(queries, self.q.keys, self.q.values, self.q.offset, scale)
 

@@ -374,15 +374,15 @@ def q8_prefill_attention(q, keys, values, n, scale):
 
     q [B, Hq, L, 128] for the chunk's positions n-L .. n-1, whose K/V are already the last L of
     the first ``n`` cache rows; row i sees keys 0 .. n-L+i. Any L >= 1. Chunks of more than 16
-    rows run the prefill kernel (256 query rows per workgroup over shared K/V tiles: dequantized to
-    fp16 for 1, 2, 4 and 8 query heads per KV head, the exact codes for other groupings), up to 16
-    the verify kernel. Returns [B, Hq, L, 128] in q's dtype."""
+    rows, or of more than 64 query rows per KV head, run the prefill kernel (256 query rows per workgroup over shared K/V tiles: dequantized to
+    fp16 for 1, 2, 4 and 8 query heads per KV head, the exact codes for other groupings), smaller
+    ones the verify kernel. Returns [B, Hq, L, 128] in q's dtype."""
     B, Hq, L, D = q.shape
     kc, ks, kb = keys
     Hkv = kc.shape[1]
     if D != 128 or Hkv < 1 or Hq % Hkv:
         raise ValueError("prefill needs head_dim 128 and Hq a multiple of Hkv")
-    if L <= 16:
+    if L <= 16 and Hq // Hkv * L <= 64:
         return q8_verify_attention(q, keys, values, n, scale)
     if Hq // Hkv > 64:
         raise ValueError(f"{Hq // Hkv} query heads per KV head exceed 64")

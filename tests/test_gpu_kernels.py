@@ -1007,6 +1007,32 @@ def test_dequantize_kv_bit_exact(dev, bits, gs, D, n, cap, B, H):
         assert torch.equal(dequantize(*buf, gs, bits, n=n), want)
 
 
+@pytest.mark.parametrize("G,Hkv,L", [(6, 2, 10), (6, 2, 11), (6, 2, 16), (8, 2, 9), (8, 1, 16), (64, 1, 2),
+                                     (33, 1, 2)])
+def test_blocks_of_more_than_64_query_rows_per_kv_head(dev, G, Hkv, L):
+    """Blocks of up to 16 rows whose query rows per KV head exceed the verify kernel's 64 go through the
+    prefill kernel (one row less than the limit, 60, through the verify kernel): the cache's protocol and
+    the function against the oracle, the appended rows against a plain append."""
+    from lagunalab_amd.cache import DequantKVCache, QuantizedKVCache
+    from lagunalab_amd.q8_attn import q8_prefill_attention
+    rng = np.random.default_rng(G + L)
+    n = 700
+    k, v = (to_dev_bf16(Q.randn_bf16(rng, (1, Hkv, n + L, 128)), dev) for _ in range(2))
+    q = Q.randn_bf16(rng, (1, Hkv * G, L, 128))
+    cache, plain = DequantKVCache(fused_decode=True), QuantizedKVCache()
+    cache.update_and_fetch(k[:, :, :n], v[:, :, :n])
+    plain.update_and_fetch(k[:, :, :n], v[:, :, :n])
+    cache.update_and_fetch(k[:, :, n:], v[:, :, n:])
+    plain.update_and_fetch(k[:, :, n:], v[:, :, n:])
+    out = cache.attend(to_dev_bf16(q, dev), 0.09)
+    for a, b in zip((*cache.q.keys, *cache.q.values), (*plain.keys, *plain.values)):
+        assert torch.equal(a[:, :, :n + L], b[:, :, :n + L])
+    want = A.fused_attention(q, cache_np(plain.keys), cache_np(plain.values), n + L, 0.09, causal=True)
+    assert_attn_close(out, want, "attend")
+    assert_attn_close(q8_prefill_attention(to_dev_bf16(q, dev), plain.keys, plain.values, n + L, 0.09),
+                      want, "function")
+
+
 @pytest.mark.parametrize("L", [1, 3])
 def test_rows_stay_pending_when_attend_raises(dev, L):
     """attend() refusing its queries (7 heads over 2 KV heads) leaves the step's rows pending: the next
