@@ -156,13 +156,16 @@ __global__ __launch_bounds__(256) void quantize_group_kernel(
   }
 }
 
-// The first n rows of every head, of one or two caches of one shape (K and V in one launch). A
-// head's rows are contiguous on both sides, so element e of a head's n x D is element e of its
-// output and a workgroup needs one division (its head); a thread takes DQ_ITER runs of 8 elements
-// (8 divides every group size), 256 runs apart, all loads before the first store. Bound by its traffic: a
-// token's append and 32,769 rows x 8 heads x 128 of K and V (205 MB read and written; a large copy runs at 4.7-5.2
-// TB/s) take 49 us, with a launch each, 64-bit divisions per run and one run per thread 56.
+// The first n rows of every head, of one or two caches of one shape (grid.y: K and V in one launch). A
+// thread takes DQ_ITER runs of 8 elements (8 divides every group size), 256 runs apart, all loads
+// before the first store. The runs are numbered through over the heads, as the output holds them: one
+// division per run (its head, for the input side) and no workgroup that is part empty, however short
+// the heads. Bound by its traffic: a token's append and 32,769 rows x 8 heads x 128 of K and V (205 MB
+// read and written; a large copy runs at 4.7-5.2 TB/s) take 48 us, with a launch each, 64-bit divisions
+// per run and one run per thread 56. 65,536 heads of one row 7.1 us, 32,768 of 65 rows 150 (workgroups
+// of whole heads 33 and 259, the 64-bit divisions 8.4 and 161).
 constexpr int DQ_ITER = 4;
+constexpr int64_t DQ_RUNS = ((int64_t)1 << 31) - 256 * DQ_ITER;  // of one launch: 32-bit run numbers
 struct DequantTarget {
   const uint8_t* codes;
   const uint16_t* scales;
@@ -172,34 +175,28 @@ struct DequantTarget {
 
 template <int BITS>
 __global__ __launch_bounds__(256) void dequantize_kernel(DequantTarget ta, DequantTarget tb,
-                                                         uint32_t wgs_per_head, uint32_t BH,
-                                                         int64_t head_in, int64_t head_out,
+                                                         uint32_t runs, uint32_t runs_per_head,
+                                                         FastDiv per_head, int64_t head_in,
                                                          int gs_shift) {
-  uint32_t hd = blockIdx.x / wgs_per_head;
-  const int64_t e0 = ((int64_t)(blockIdx.x - hd * wgs_per_head) * (256 * DQ_ITER) + threadIdx.x) * 8;
-  const bool second = hd >= BH;  // workgroup-uniform
-  if (second) hd -= BH;
-  const DequantTarget t = second ? tb : ta;
-  const int64_t in0 = hd * head_in;  // elements before this head's rows
-  const uint8_t* codes = t.codes + in0 * BITS / 8;
-  const uint16_t* scales = t.scales + (in0 >> gs_shift);
-  const uint16_t* biases = t.biases + (in0 >> gs_shift);
-  uint16_t* out = t.out + hd * head_out;
+  const DequantTarget t = blockIdx.y ? tb : ta;
+  const uint32_t i0 = blockIdx.x * (256 * DQ_ITER) + threadIdx.x;
   uint2 w[DQ_ITER];
   uint16_t sc[DQ_ITER], bi[DQ_ITER];
 #pragma unroll
   for (int k = 0; k < DQ_ITER; ++k) {
-    const int64_t e = e0 + k * (256 * 8);
-    if (e >= head_out) continue;
-    if (BITS == 8) w[k] = *reinterpret_cast<const uint2*>(codes + e);
-    else w[k].x = *reinterpret_cast<const uint32_t*>(codes + e / 2);
-    sc[k] = scales[e >> gs_shift];
-    bi[k] = biases[e >> gs_shift];
+    const uint32_t i = i0 + 256 * k;
+    if (i >= runs) continue;
+    const uint32_t hd = fdiv_u(i, per_head);
+    const int64_t e = hd * head_in + (int64_t)(i - hd * runs_per_head) * 8;
+    if (BITS == 8) w[k] = *reinterpret_cast<const uint2*>(t.codes + e);
+    else w[k].x = *reinterpret_cast<const uint32_t*>(t.codes + e / 2);
+    sc[k] = t.scales[e >> gs_shift];
+    bi[k] = t.biases[e >> gs_shift];
   }
 #pragma unroll
   for (int k = 0; k < DQ_ITER; ++k) {
-    const int64_t e = e0 + k * (256 * 8);
-    if (e >= head_out) continue;
+    const uint32_t i = i0 + 256 * k;
+    if (i >= runs) continue;
     const float s = bf16_to_f32(sc[k]), b = bf16_to_f32(bi[k]);
     uint32_t o[4];
 #pragma unroll
@@ -216,7 +213,7 @@ __global__ __launch_bounds__(256) void dequantize_kernel(DequantTarget ta, Dequa
       o[j] = (uint32_t)f32_to_bf16(__fadd_rn(__fmul_rn(s, (float)c0), b)) |
              ((uint32_t)f32_to_bf16(__fadd_rn(__fmul_rn(s, (float)c1), b)) << 16);
     }
-    *reinterpret_cast<uint4*>(out + e) = make_uint4(o[0], o[1], o[2], o[3]);
+    reinterpret_cast<uint4*>(t.out)[i] = make_uint4(o[0], o[1], o[2], o[3]);
   }
 }
 
@@ -230,14 +227,25 @@ int dequantize(DequantTarget a, DequantTarget b, int two, int64_t B, int64_t H, 
   LQ_CHECK_ARG(a.codes && a.scales && a.biases && a.out, "null pointer");
   LQ_CHECK_ARG(!two || (b.codes && b.scales && b.biases && b.out), "null pointer");
   if (n == 0) return LQ_OK;
-  const int64_t per_head = (n * D / 8 + 256 * DQ_ITER - 1) / (256 * DQ_ITER);
-  const int64_t wgs = (two ? 2 : 1) * B * H * per_head;
-  LQ_CHECK_ARG(wgs < (int64_t)1 << 31, "dequantization of %lld values is too large for one call",
-               (long long)(B * H * n * D));
+  // launches of at most DQ_RUNS runs: all heads at once but for outputs of 32 GB and more
   const int shift = group_size == 32 ? 5 : group_size == 64 ? 6 : 7;
-  (bits == 8 ? dequantize_kernel<8> : dequantize_kernel<4>)<<<dim3((unsigned)wgs), dim3(256), 0, st>>>(
-      a, b, (uint32_t)per_head, (uint32_t)(B * H), cap * D, n * D, shift);
-  LQ_CHECK_LAUNCH("dequantize_kernel");
+  const int64_t BH = B * H, rows = std::min(n, std::max<int64_t>(1, DQ_RUNS / (D / 8)));
+  LQ_CHECK_ARG(D / 8 <= DQ_RUNS, "rows of %lld values", (long long)D);
+  const int64_t heads = rows < n ? 1 : std::min(BH, std::max<int64_t>(1, DQ_RUNS / (n * D / 8)));
+  for (int64_t h = 0; h < BH; h += heads)
+    for (int64_t r = 0; r < n; r += rows) {
+      const int64_t nh = std::min(heads, BH - h), nr = std::min(rows, n - r);
+      const int64_t in = (h * cap + r) * D, out = (h * n + r) * D;
+      auto part = [&](const DequantTarget& t) {
+        return DequantTarget{t.codes + in * bits / 8, t.scales + (in >> shift),
+                             t.biases + (in >> shift), t.out + out};
+      };
+      const uint32_t per_head = (uint32_t)(nr * D / 8), runs = (uint32_t)nh * per_head;
+      const dim3 grid((runs + 256 * DQ_ITER - 1) / (256 * DQ_ITER), two ? 2 : 1);
+      (bits == 8 ? dequantize_kernel<8> : dequantize_kernel<4>)<<<grid, dim3(256), 0, st>>>(
+          part(a), part(b), runs, per_head, make_fastdiv(per_head), cap * D, shift);
+      LQ_CHECK_LAUNCH("dequantize_kernel");
+    }
   return LQ_OK;
 }
 

@@ -1048,3 +1048,24 @@ def test_rows_stay_pending_when_attend_raises(dev, L):
         cache.attend(torch.zeros((1, 7, L, 128), dtype=torch.bfloat16, device=dev), 0.09)
     for a, b in zip(cache.state[0] + cache.state[1], plain.state[0] + plain.state[1]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("bits,gs,D,n,cap,B,H", [(8, 64, 128, 1, 1, 8, 512), (8, 32, 96, 1, 3, 5, 333),
+                                                 (4, 128, 128, 3, 7, 16, 100), (8, 64, 64, 65, 70, 2, 301)])
+def test_dequantize_of_many_short_heads(dev, bits, gs, D, n, cap, B, H):
+    """Heads shorter than a workgroup's 8,192 elements, several to a workgroup and across its edges."""
+    from lagunalab_amd.quant import dequantize, dequantize_kv
+    g = torch.Generator(device="cpu").manual_seed(n + D)
+    bufs = []
+    for _ in range(2):
+        c = torch.randint(0, 256, (B, H, cap, D * bits // 8), generator=g, dtype=torch.uint8).to(dev)
+        bufs.append((c, *(torch.randn((B, H, cap, D // gs), generator=g).to(torch.bfloat16).to(dev)
+                          for _ in range(2))))
+    for got, buf in zip(dequantize_kv(*bufs, gs, bits, n), bufs):
+        codes, s, b = (t[:, :, :n] for t in buf)
+        if bits == 4:
+            codes = torch.stack([codes & 15, codes >> 4], -1).reshape(B, H, n, D)
+        want = (codes.float() * s.float().repeat_interleave(gs, -1)
+                + b.float().repeat_interleave(gs, -1)).to(torch.bfloat16)
+        assert torch.equal(got, want)
+        assert torch.equal(dequantize(*buf, gs, bits, n=n), want)
