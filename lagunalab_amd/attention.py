@@ -89,27 +89,59 @@ def _sdpa(q, k, v, mask, scale):
     return torch.matmul(p, v.float()).reshape(B, Hq, Lq, D).to(q.dtype)
 
 
-def _unwatched(*tensors):
+# looked up once: the checks run on every product of a short block, which the host bounds
+_C = torch._C
+_peek_functorch, _is_tracing, _is_compiling = (_C._functorch.peek_interpreter_stack, _C._is_tracing,
+                                               torch.compiler.is_compiling)
+_dispatch_modes, _function_modes = _C._len_torch_dispatch_stack, _C._len_torch_function_stack
+_autocast, _grad_enabled, _Tensor = _C._is_any_autocast_enabled, torch.is_grad_enabled, torch.Tensor
+
+
+def _unwatched(x, w):
     """Whether an operation on these may be launched past torch's dispatcher: plain tensors, and nothing
     that records, rewrites or casts what the dispatcher sees -- autograd, forward mode, function
     transforms (vmap, grad), jit and fx tracing, compilation, dispatch and function modes (other than a
     default device's) and autocast. Those get the library product, which they can see."""
-    return (all(type(t) is torch.Tensor for t in tensors)
-            and not (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
-            and forward_ad._current_level < 0
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and not torch._C._is_tracing() and not torch.compiler.is_compiling()
-            and torch._C._len_torch_dispatch_stack() == 0
-            and all(type(torch._C._get_function_stack_at(i)) is DeviceContext
-                    for i in range(torch._C._len_torch_function_stack()))
-            and not torch.is_autocast_enabled(tensors[0].device.type))
+    return (type(x) is type(w) is _Tensor
+            and not ((x.requires_grad or w.requires_grad) and _grad_enabled())
+            and not _dispatch_modes() and _peek_functorch() is None and not _is_tracing()
+            and forward_ad._current_level < 0 and not _autocast() and not _is_compiling()
+            and (not _function_modes() or all(type(_C._get_function_stack_at(i)) is DeviceContext
+                                              for i in range(_function_modes()))))
+
+
+def _row_form_pays(rows, N, K):
+    """Whether ``lq_gemm_rows_bf16`` is the faster of the two for ``rows`` x K against N outputs. A wave
+    has an eighth of K in steps of 32, eight of them in flight, so up to 2,048 it is one round of loads
+    and to 4,096 two (worth it from the second's half); a workgroup has 16 outputs, so up to 4,096 there
+    is one on each of the 256 CUs, and every workgroup reads all rows. us per call, row form / library,
+    weights not cached, in a graph:
+
+    * one workgroup per CU -- 1,024 outputs of 1,024, 16 rows 5.7 / 5.8; 2,048 of 4,096, 8 rows 8.3 /
+      14.3, 16 rows 9.7 / 14.3; 4,096 of 3,072, 16 rows 10.5 / 12.6. Not with a second round hardly
+      used (1,024 of 2,304, 8 rows 7.8 / 7.6) or three (2,048 of 6,144, 8 rows 11.4 / 11.0; 1,024 of
+      5,120, 16 rows 14.3 / 9.9), nor with short rows (512 of 512, 8 rows 4.8 / 4.4);
+    * two -- 6,176 of 2,048, 8 rows 8.8 / 12.4; 8,192 of 1,536, 12 rows 10.2 / 10.7, 16 rows 11.2 / 10.6;
+      6,176 of 1,024, 5 rows 7.7 / 8.1, 8 rows 8.3 / 8.2; with two rounds 6,176 of 4,096, 8 rows 15.0 /
+      14.3;
+    * three, all eight steps of a round used -- 8,240 of 2,048, 8 rows 11.2 / 12.9; 12,288 of 1,920, 8
+      rows 12.7 / 13.4, 12 rows 14.3 / 13.5; 10,240 of 1,792, 8 rows 13.0 / 12.6; 16,384 of 1,920, 8
+      rows 16.5 / 14.8."""
+    if N < 1024 or not (1024 <= K <= 2048 or 3072 <= K <= 4096):
+        return False
+    if N <= 4096:
+        return True
+    if K > 2048:
+        return False
+    if N <= 8192:
+        return rows <= (12 if K >= 1536 else 4)
+    return N <= 12288 and K > 1792 and rows <= 8
 
 
 def _row_form(x, w, rows, K):
     """Whether ``lq_gemm_rows_bf16`` takes this product: what the kernel reads (bf16, contiguous,
     16-byte aligned), in a call that nothing watches."""
-    return (K <= (4096 if rows > 8 else 6144) and K % 8 == 0
-            and w.dim() == 2 and w.shape[1] == K and w.shape[0] > 0
+    return (w.dim() == 2 and w.shape[1] == K and K % 8 == 0 and _row_form_pays(rows, w.shape[0], K)
             and x.dtype == w.dtype == torch.bfloat16 and x.is_cuda and x.device == w.device
             and x.is_contiguous() and w.is_contiguous() and _unwatched(x, w)
             and (x.data_ptr() | w.data_ptr()) % 16 == 0)
@@ -118,10 +150,7 @@ def _row_form(x, w, rows, K):
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """``x @ w.T`` for bf16 ``x [..., K]`` and ``w [N, K]``: one row (a decode step) runs
     ``lq_gemv_bf16`` (weight-streaming, HBM-bound), 2 to 16 rows (a verify block) the matrix-core
-    form of it, ``lq_gemm_rows_bf16``, more rows the library GEMM. Every workgroup of the row form
-    reads all of x, so long rows go to the library where that costs more than its tiling: us per
-    call, row form / library, 2,048 outputs: 16 x 4,096 9.4 / 11.6, 8 x 6,144 11.8 / 11.7, 16 x
-    6,144 13.9 / 11.5; 6,176 outputs of 2,048: 2 rows 7.8 / 12.6, 8 9.4 / 12.9, 16 11.1 / 12.7."""
+    form of it, ``lq_gemm_rows_bf16``, where it is faster, more rows the library GEMM."""
     K = x.shape[-1]
     rows = x.numel() // K if K else 0
     if rows != 1 and not (2 <= rows <= 16 and _row_form(x, w, rows, K)):

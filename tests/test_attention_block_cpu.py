@@ -111,3 +111,13 @@ def test_unwatched_calls_only_outside_tracing_modes_and_autocast():
     with forward_ad.dual_level():
         call(forward_ad.make_dual(x, x))
     assert len(seen) >= 10 and not any(seen)
+
+
+@pytest.mark.parametrize("rows,N,K,pays", [
+    (2, 1023, 2048, 0), (2, 1024, 1023, 0), (16, 1024, 1024, 1), (16, 4096, 2048, 1), (16, 2048, 2049, 0),
+    (16, 2048, 3072, 1), (16, 4096, 4096, 1), (2, 2048, 4097, 0), (2, 4097, 3072, 0), (12, 4097, 1536, 1),
+    (13, 8192, 2048, 0), (4, 8192, 1535, 1), (5, 8192, 1535, 0), (8, 8193, 1793, 1), (8, 8193, 1792, 0),
+    (9, 8193, 2048, 0), (8, 12289, 2048, 0)])
+def test_row_form_only_where_it_was_measured_faster(rows, N, K, pays):
+    from lagunalab_amd.attention import _row_form_pays
+    assert _row_form_pays(rows, N, K) == bool(pays)

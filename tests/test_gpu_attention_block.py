@@ -528,11 +528,16 @@ def test_gemm_rows(dev, M, N, K):
     """The projections of 2 to 16 rows: outputs past a 16-column tile, K that leaves waves empty or
     with part of a step. Against float64 on the same bf16 values: half a bf16 step of the result and
     the fp32 sums' own error (K terms of 2^-24 of their absolute sum)."""
-    from lagunalab_amd.attention import linear
+    from lagunalab_amd import _lib
+    lib = _lib.load()
     g = torch.Generator(device="cpu").manual_seed(M + N + K)
     x = torch.randn((1, M, K), generator=g).to(torch.bfloat16)
     w = (torch.randn((N, K), generator=g) * 0.05).to(torch.bfloat16)
-    got = linear(x.to(dev), w.to(dev)).double().cpu()
+    xd, wd = x.to(dev), w.to(dev)
+    y = torch.empty((1, M, N), dtype=torch.bfloat16, device=dev)
+    _lib.check(lib.lq_gemm_rows_bf16(wd.data_ptr(), xd.data_ptr(), y.data_ptr(), M, N, K,
+                                     _lib.stream_ptr(dev)), "lq_gemm_rows_bf16")
+    got = y.double().cpu()
     want = x.double() @ w.double().t()
     bound = want.abs() * 2.0 ** -8 + (x.double().abs() @ w.double().abs().t()) * K * 2.0 ** -24
     assert got.shape == (1, M, N) and bool(((got - want).abs() <= bound).all())
@@ -545,7 +550,7 @@ def test_row_products_are_seen_by_tracing_modes_and_autocast(dev):
     from torch.utils.flop_counter import FlopCounterMode
     from lagunalab_amd.attention import linear
     g = torch.Generator(device="cpu").manual_seed(4)
-    w = torch.randn((256, 1024), generator=g).to(torch.bfloat16).to(dev)
+    w = torch.randn((1024, 1024), generator=g).to(torch.bfloat16).to(dev)
     x, x2 = (torch.randn((4, 1024), generator=g).to(torch.bfloat16).to(dev) for _ in range(2))
     want = torch.matmul(x2, w.t())
     traced = torch.jit.trace(lambda a: linear(a, w), (x,), check_trace=False)
@@ -553,6 +558,28 @@ def test_row_products_are_seen_by_tracing_modes_and_autocast(dev):
     assert torch.equal(make_fx(lambda a: linear(a, w))(x)(x2), want)
     with FlopCounterMode(display=False) as flops:
         linear(x, w)
-    assert flops.get_total_flops() == 2 * 4 * 256 * 1024
+    assert flops.get_total_flops() == 2 * 4 * 1024 * 1024
     with torch.autocast("cuda", dtype=torch.float16):
         assert linear(x, w).dtype == torch.float16
+
+
+@pytest.mark.parametrize("M,N,K,row_form", [(2, 1024, 1024, True), (16, 2048, 4096, True), (8, 6176, 2048, True),
+                                            (13, 6176, 2048, False), (8, 8240, 2048, True),
+                                            (8, 2048, 6144, False), (5, 1000, 2048, False)])
+def test_linear_takes_the_row_form_where_it_is_faster(dev, M, N, K, row_form):
+    """linear() on both sides of the rule's lines: the kernel that runs, and its result against float64
+    (half a bf16 step and the fp32 sums' error)."""
+    from lagunalab_amd.attention import linear
+    g = torch.Generator(device="cpu").manual_seed(M + N + K)
+    x = torch.randn((1, M, K), generator=g).to(torch.bfloat16)
+    w = (torch.randn((N, K), generator=g) * 0.05).to(torch.bfloat16)
+    xd, wd = x.to(dev), w.to(dev)
+    linear(xd, wd)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        got = linear(xd, wd)
+        torch.cuda.synchronize()
+    names = [e.key for e in prof.key_averages()]
+    assert names and any("gemm_rows_kernel" in n for n in names) == row_form, names
+    want = x.double() @ w.double().t()
+    bound = want.abs() * 2.0 ** -8 + (x.double().abs() @ w.double().abs().t()) * K * 2.0 ** -24
+    assert bool(((got.double().cpu() - want).abs() <= bound).all())
