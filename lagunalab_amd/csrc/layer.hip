@@ -651,10 +651,6 @@ int gate_heads(const uint16_t* attn, const uint16_t* gate, int64_t gate_stride, 
   LQ_CHECK_ARG(D == ND, "head_dim must be 128 (got %lld)", (long long)D);
   LQ_CHECK_ARG(B >= 1 && Hq >= 1 && L >= 1, "bad shape");
   LQ_CHECK_ARG(attn && gate && out && attn != out, "null or aliased pointer");
-  LQ_CHECK_ARG(gate_stride >= (per_dim ? Hq * D : Hq) &&
-                   (!per_dim || (gate_stride % 8 == 0 && ((uintptr_t)gate & 15) == 0)),
-               "a per-dim gate needs 16-byte aligned rows of at least Hq x 128 (stride %lld)",
-               (long long)gate_stride);
   const int64_t total = B * Hq * L * (ND / 8);
   LQ_CHECK_ARG(total / 256 < (int64_t)INT32_MAX, "too many rows");
   gate_heads_kernel<<<dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st>>>(
@@ -675,8 +671,13 @@ extern "C" int lq_gate_heads(const uint16_t* attn, const uint16_t* gate, uint16_
 extern "C" int lq_gate_heads_strided(const uint16_t* attn, const uint16_t* gate,
                                      int64_t gate_stride, uint16_t* out, int64_t B, int64_t Hq,
                                      int64_t L, int64_t D, int per_dim, void* stream) {
-  lq::clear_error();
-  return lq::gate_heads(attn, gate, gate_stride, out, B, Hq, L, D, per_dim, (hipStream_t)stream);
+  using namespace lq;
+  clear_error();
+  LQ_CHECK_ARG(gate_stride >= (per_dim ? Hq * D : Hq) &&
+                   (!per_dim || (gate_stride % 8 == 0 && ((uintptr_t)gate & 15) == 0)),
+               "a per-dim gate needs 16-byte aligned rows of at least Hq x 128 (stride %lld)",
+               (long long)gate_stride);
+  return gate_heads(attn, gate, gate_stride, out, B, Hq, L, D, per_dim, (hipStream_t)stream);
 }
 
 extern "C" int lq_qkv_norm_rope(const uint16_t* proj, int64_t N, uint16_t* q_out, uint16_t* k_out,

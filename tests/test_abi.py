@@ -195,3 +195,17 @@ def test_workspace_size_never_falls_as_the_length_grows(lib, kind, Hq, Hkv):
             continue
         vs = [lib.lq_verify_workspace_bytes(1, Hq, Hkv, L, 128, n) for n in lengths if n >= L]
         assert all(a <= b for a, b in zip(vs, vs[1:])), (L, vs)
+
+
+@pytest.mark.skipif(__import__("torch").cuda.is_available(), reason="host pointers: stops at the launch")
+def test_gate_heads_takes_any_gate_address(lib):
+    """The contiguous gate's entry has no rule on the gate's address (without a GPU the call gets as far
+    as its launch); the strided one asks for 16-byte aligned rows."""
+    import ctypes as C
+    from lagunalab_amd import _lib
+    buf = (C.c_char * 65536)()
+    p = (C.addressof(buf) + 63) // 64 * 64
+    args = (p + 16384, 1, 2, 1, 128, 1, None)
+    assert lib.lq_gate_heads(p, p + 8194, *args) == _lib.LQ_EHIP
+    assert lib.lq_gate_heads_strided(p, p + 8194, 256, *args) == _lib.LQ_EINVAL
+    assert lib.lq_gate_heads_strided(p, p + 8192, 256, *args) == _lib.LQ_EHIP
