@@ -146,8 +146,10 @@ class QuantizedKVCache:
 class _PendingRows(tuple):
     """The ``(codes, scales, biases)`` views returned on a fused single-token step. The new row
     is quantized and written by the following ``attend`` (one fused kernel with the attention);
-    any use of this tuple first completes the append, so its contents are always the reference's.
-    The views themselves are made on first use: a decode loop never looks at them, and the six
+    every Python-level use of this tuple (indexing, iteration, unpacking, comparison, concatenation,
+    printing, copying, pickling) first completes the append, so its contents are always the
+    reference's. Not covered is C code that reads a tuple's slots without asking it (``torch.cat(p)``,
+    ``"%s" % p``): it finds None there; give it ``tuple(p)``. The views themselves are made on first use: a decode loop never looks at them, and the six
     slices were a quarter of a short step, which the host bounds (a token at 1,038 keys, 32/8 heads:
     26.8 -> 19.6 us; at 32,772 keys, 48/8: 27.0 -> 20.0)."""
 
@@ -179,6 +181,18 @@ class _PendingRows(tuple):
 
     def __ne__(self, other):
         return not self == other
+
+    def __lt__(self, other):
+        return self._items() < (tuple(other) if isinstance(other, tuple) else other)
+
+    def __le__(self, other):
+        return self._items() <= (tuple(other) if isinstance(other, tuple) else other)
+
+    def __gt__(self, other):
+        return self._items() > (tuple(other) if isinstance(other, tuple) else other)
+
+    def __ge__(self, other):
+        return self._items() >= (tuple(other) if isinstance(other, tuple) else other)
 
     def __hash__(self):
         return hash(self._items())

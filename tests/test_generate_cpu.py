@@ -104,8 +104,8 @@ def test_greedy_stops_at_eos(model):
 
 
 def test_pending_rows_behave_as_the_tuple_of_views():
-    """The tuple of a fused step makes its views on first use: every way of reading it completes the
-    append first and gives the views of the step's own buffers and length, also after the cache has
+    """The tuple of a fused step makes its views on first use: every Python-level way of reading it
+    completes the append first and gives the views of the step's own buffers and length, also after the cache has
     grown or been trimmed."""
     import copy
     from lagunalab_amd.cache import _PendingRows
@@ -130,3 +130,15 @@ def test_pending_rows_behave_as_the_tuple_of_views():
     p = _PendingRows(bufs, 3, Cache())
     assert p == p and p[0] is p[0] and p[0] in p and p.index(p[0]) == 0 and hash(p) == hash(tuple(p))
     assert "tensor" in repr(p)
+    # ordering compares the views (here the first ones, of one value each), on either side
+    ones = tuple(torch.full((1, 1, 4, 1), float(i)) for i in range(3))
+    more = (ones[0][:, :, :1] + 1,) + ones[1:]
+    for cmp in (lambda a: a < more, lambda a: a <= more, lambda a: more > a, lambda a: more >= a):
+        c = Cache()
+        assert cmp(_PendingRows(ones, 1, c)) and c.flushed > 0
+    for cmp in (lambda a: a > more, lambda a: a >= more, lambda a: more < a, lambda a: more <= a):
+        c = Cache()
+        assert not cmp(_PendingRows(ones, 1, c)) and c.flushed > 0
+    # what a tuple's C readers need
+    c = Cache()
+    assert torch.cat(tuple(_PendingRows(bufs, 3, c)), -1).shape == (1, 2, 3, 9) and c.flushed > 0
