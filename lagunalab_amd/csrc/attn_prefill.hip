@@ -926,18 +926,27 @@ __global__ __launch_bounds__(64 * PW, 1) void q8_prefill_kernel(
 // workgroup per 2 rows of a block; a row's parts (those of consecutive shares) are dealt to four
 // groups of 32 lanes (4 dims each), which combine through LDS. Blocks that one share covered whole
 // are written already. Bound by the loads' latency: 33 MB of parts (64 rows at 82,735 keys, 32/8
-// heads, 21 parts per row) took 20.4 us with one group per row and 8 rows per workgroup.
+// heads, 31 parts per row) took 20.4 us with one group per row and 8 rows per workgroup. The tiles
+// before the block are summed by all threads: in a loop of each, that was most of the launch where
+// blocks are many (3,072 rows behind 2,000 keys, 32/8 heads, split into parts: 336 us in all, now 243).
 __global__ __launch_bounds__(256) void prefill_merge_kernel(uint16_t* __restrict__ out, int n, int L,
                                                             int Hkv, int G, PrefillSplit sp) {
   __shared__ f4_t sh_acc[2][4][32];
   __shared__ float2 sh_ml[2][4];
+  __shared__ int sh_u[4];
   const int hk = blockIdx.y % Hkv, b = blockIdx.y / Hkv;
   const int R = L * G, base = n - L;
   const int pb = blockIdx.x / (PROWS / 2);
   const int tr = threadIdx.x >> 7, grp = (threadIdx.x >> 5) & 3, ln = threadIdx.x & 31;
   const int wrow = 2 * (blockIdx.x % (PROWS / 2)) + tr;
-  int u0 = 0;
-  for (int j = 0; j < pb; ++j) u0 += prefill_tiles(j, R, sp.g, base);
+  // tiles of the blocks before this one, over the workgroup's threads
+  int part = 0;
+  for (int j = threadIdx.x; j < pb; j += 256) part += prefill_tiles(j, R, sp.g, base);
+#pragma unroll
+  for (int m = 1; m < 64; m *= 2) part += __shfl_xor(part, m);
+  if ((threadIdx.x & 63) == 0) sh_u[threadIdx.x >> 6] = part;
+  __syncthreads();
+  const int u0 = sh_u[0] + sh_u[1] + sh_u[2] + sh_u[3];
   const int u1 = u0 + prefill_tiles(pb, R, sp.g, base);
   const int j0 = u0 / sp.tiles, j1 = (u1 - 1) / sp.tiles;
   const int f = pb * PROWS + wrow;
