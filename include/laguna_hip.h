@@ -317,8 +317,9 @@ int lq_q8_prefill_attn(const uint16_t* q, const uint8_t* kc, const uint16_t* ks,
                        float scale, uint16_t* out, void* stream);
 
 /*
- * lq_q8_prefill_attn for any grouping of up to 64 query heads per KV head. Chunks whose blocks of
- * 256 rows would leave CUs idle have their keys split over workgroups; the partial rows need
+ * lq_q8_prefill_attn for any grouping of up to 64 query heads per KV head. Where that is faster than
+ * whole blocks of 256 rows (few blocks for the CUs, or a last round of blocks that leaves many of
+ * them idle) the keys are split over workgroups; the partial rows need
  * lq_prefill_workspace_bytes of scratch (0 for chunks that are not split; negative on bad
  * arguments; at most about 70 MB), of any contents and free again when the call's work is done.
  */

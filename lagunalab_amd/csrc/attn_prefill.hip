@@ -1002,29 +1002,44 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(uint16_t* __restrict
 
 // How the blocks of a chunk are dealt to workgroups: whole, one block each (tiles 0), or each KV
 // head's tiles, block after block, in equal shares of `tiles` for as many workgroups as fill the
-// CUs. Costs in tiles (3.7-4.2 us each, by clock): whole blocks go round by round, longest first;
-// a share pays about two per block that it touches (q, the first copies, the output rows) and the
-// partial rows with their merge launch about six. Measured, us per 32/8 chunk, whole against
-// split: 64 rows at 82,735 keys 2,068 / 137, 1,024 rows at 83,695 keys 2,138 / 1,440; 48/8, 512
-// rows at 8,193 keys, 237 / 147, 2,048 rows at 62,048 keys (1.5 rounds whole) 3,908 / 3,255; and
-// where whole stays better, 2,048 rows at 2,112 keys (17 tiles at most) 79 / 120.
-constexpr int SEGMENT_TILES = 2;
-constexpr int MERGE_TILES = 6;
-constexpr int MIN_SHARE = 4;
+// CUs. Whole blocks go round by round, longest first: their time follows the tiles of each round's
+// longest block. A share's time follows its tiles, the blocks that it touches (q, the first copies,
+// the output rows) and the partial rows that are written and merged. Costs fitted to 190 chunks timed
+// both ways (G 1 to 8, 17 to 4,096 rows behind 64 to 32,000 keys; within 15% from 40 us on); split where
+// they say 3% or more. us, whole / split: 32/8 heads, 64 rows behind 32,000 keys 790 / 56, 512 behind
+// 1,000 48 / 53 and 2,000 73 / 60, 1,536 behind 2,000 100 / 115, 3,072 behind 2,000 190 / 242; 16/2,
+// 2,048 behind 500 74 / 80 and 2,000 111 / 95; 48/8, 512 behind 500 61 / 65 and 8,000 419 / 196, 2,048
+// behind 2,000 293 / 312 and 16,000 1,628 / 1,305.
+struct SplitCosts {  // in 10 ns
+  int tile, segment, block, split;  // of a share per tile and touched block, of all blocks each, constant
+  int whole_tile, whole;            // of whole blocks per tile, constant
+};
+constexpr SplitCosts FP16_COSTS = {390, 900, 17, 900, 308, 990};
+constexpr SplitCosts CODES_COSTS = {600, 700, 27, 500, 564, 920};
+constexpr int MIN_SHARE = 2;
+
+// Groupings that the verify kernel served before keep its arithmetic (see the top of the file).
+bool codes_variant(int64_t G) { return !(G == 1 || G == 2 || G == 4 || G == 8); }
+
 PrefillSplit plan_split(int64_t B, int64_t Hkv, int64_t G, int64_t L, int64_t n, int cus) {
   const int R = (int)(L * G), base = (int)(n - L), npb = (R + PROWS - 1) / PROWS;
   PrefillSplit sp{make_fastdiv((uint32_t)G), npb, 0, nullptr, nullptr};
   const int64_t S = cus / (B * Hkv);
   if (S < 2 || npb > 4 * S) return sp;  // no CUs to spare; the last round matters little
   int64_t total = 0, rounds = 0;
-  for (int pb = 0; pb < npb; ++pb) {
-    const int t = prefill_tiles(pb, R, sp.g, base);
+  for (int i = 0, r = -1; i < npb; ++i) {  // longest blocks first, B Hkv of each length
+    const int t = prefill_tiles(npb - 1 - i, R, sp.g, base);
     total += t;
-    if ((npb - 1 - pb) % S == 0) rounds += t;
+    if ((int)(((i + 1) * B * Hkv - 1) / cus) > r) {
+      rounds += t;
+      ++r;
+    }
   }
   const int64_t tiles = std::max<int64_t>(MIN_SHARE, (total + S - 1) / S);
   const int64_t touched = 2 + (tiles - 2) / prefill_tiles(0, R, sp.g, base);  // block 0: shortest
-  if (33 * (tiles + SEGMENT_TILES * touched + MERGE_TILES) > 32 * rounds) return sp;  // 3% or more
+  const SplitCosts c = codes_variant(G) ? CODES_COSTS : FP16_COSTS;
+  const int64_t split = c.tile * tiles + c.segment * touched + c.block * npb * B * Hkv + c.split;
+  if (tiles >= rounds || 103 * split > 100 * (c.whole_tile * rounds + c.whole)) return sp;
   sp.tiles = (int)tiles;
   sp.shares = (int)((total + tiles - 1) / tiles);
   return sp;
@@ -1064,8 +1079,7 @@ int prefill_attn(const uint16_t* q, const uint8_t* kc, const uint16_t* ks, const
     sp.part_ml = (float2*)(sp.part_o + 2 * B * Hkv * sp.shares * PROWS * D);
   }
   const int64_t wgs = B * Hkv * sp.shares;
-  // groupings that the verify kernel served before keep its arithmetic (see the top of the file)
-  const bool codes = !(G == 1 || G == 2 || G == 4 || G == 8);
+  const bool codes = codes_variant(G);
   auto* kern = codes ? (sp.tiles ? q8_prefill_kernel<true, true> : q8_prefill_kernel<true, false>)
                      : (sp.tiles ? q8_prefill_kernel<false, true> : q8_prefill_kernel<false, false>);
   kern<<<dim3((unsigned)wgs), dim3(64 * PW), 0, st>>>(

@@ -209,3 +209,14 @@ def test_gate_heads_takes_any_gate_address(lib):
     assert lib.lq_gate_heads(p, p + 8194, *args) == _lib.LQ_EHIP
     assert lib.lq_gate_heads_strided(p, p + 8194, 256, *args) == _lib.LQ_EINVAL
     assert lib.lq_gate_heads_strided(p, p + 8192, 256, *args) == _lib.LQ_EHIP
+
+
+@pytest.mark.parametrize("Hq,Hkv,L,ctx,split", [
+    (32, 8, 64, 32000, 1), (32, 8, 512, 1000, 0), (32, 8, 512, 2000, 1), (32, 8, 1536, 2000, 0),
+    (32, 8, 3072, 2000, 0), (32, 8, 2048, 80623, 0), (16, 2, 2048, 500, 0), (16, 2, 2048, 2000, 1),
+    (48, 8, 512, 64, 0), (48, 8, 512, 7681, 1), (48, 8, 2048, 2000, 0), (48, 8, 2048, 16000, 1),
+    (96, 24, 1600, 5000, 0), (384, 64, 384, 8616, 1)])
+def test_prefill_split_where_it_was_measured_faster(lib, Hq, Hkv, L, ctx, split):
+    """Both sides of the plan's lines (on 256 CUs): chunks timed whole and split, 3% or more apart."""
+    got = lib.lq_prefill_workspace_bytes(1, Hq, Hkv, L, ctx + L)
+    assert 0 <= got <= 70 << 20 and (got > 0) == bool(split)

@@ -965,20 +965,20 @@ def test_prefill_split_passes_nan_and_infinity_on(dev, G, what):
 
 
 def test_prefill_split_shares_cover_several_blocks(dev):
-    """25 blocks per KV head on 10 workgroups each: shares of two and a half blocks (the end of one,
-    a whole one, the start of the next), against the entry that never splits."""
+    """Nine blocks per KV head on 4 workgroups each: shares of two and a quarter blocks (the end of one,
+    a whole one, the start of the next), against the verify kernel's blocks."""
     from lagunalab_amd import _lib, q8_attn
+    from lagunalab_amd.quant import quantize
     lib = _lib.load()
-    n, L, G, Hkv, B = 6600, 1600, 4, 8, 3
-    rng = np.random.default_rng(3)
-    kq, vq = make_cache(rng, B, Hkv, n, n, dev)
-    q = to_dev_bf16(Q.randn_bf16(rng, (B, Hkv * G, L, 128)), dev)
+    n, L, G, Hkv, B = 9000, 384, 6, 64, 1
+    g = torch.Generator(device=dev).manual_seed(3)
+    rnd = lambda *s: torch.randn(s, device=dev, generator=g).to(torch.bfloat16)  # noqa: E731
+    kq, vq = (quantize(rnd(B, Hkv, n, 128), 64, 8) for _ in range(2))
+    q = rnd(B, Hkv * G, L, 128)
     assert lib.lq_prefill_workspace_bytes(B, Hkv * G, Hkv, L, n) > 0
     got = q8_attn.q8_prefill_attention(q, kq, vq, n, 0.09)
-    want = torch.empty_like(q)
-    assert lib.lq_q8_prefill_attn(q.data_ptr(), *(t.data_ptr() for t in (*kq, *vq)), B, Hkv * G, Hkv,
-                                  L, 128, n, n, 0.09, want.data_ptr(), _lib.stream_ptr(dev)) == 0
-    assert_attn_close(got, want.float().cpu().numpy(), "split against whole blocks")
+    want = q8_attn._prefill_blocked(q, kq, vq, n, 0.09)
+    assert_attn_close(got, want.float().cpu().numpy(), "split against the verify kernel")
 
 
 @pytest.mark.parametrize("bits,gs,D,n,cap,B,H", [(8, 64, 128, 1, 4, 1, 1), (8, 64, 128, 65, 65, 2, 3),

@@ -219,13 +219,13 @@ def test_prefill_of_other_groupings_is_as_exact_as_the_verify_kernel(dev, G, n, 
 
 
 @pytest.mark.parametrize("G", [6, 3])
-@pytest.mark.parametrize("n,L", [(1000, 70), (3000, 70)], ids=["whole", "split"])
+@pytest.mark.parametrize("n,L", [(500, 70), (3000, 70)], ids=["whole", "split"])
 @pytest.mark.parametrize("kind", ["far keys", "large scores", "V groups", "V tiles"])
 def test_prefill_operands_far_apart(dev, kind, n, L, G):
     """What the verify kernel serves and a dequantized fp16 operand does not hold: keys 2^36 times
     others of their tile (with scores far below theirs), scores of 2^30 and more, V groups of one
-    head 2^-18 of each other, V sizes that jump by powers of two between regions of five 64-key tiles
-    (at 1,000 keys in whole blocks: the exponent changes within one walk of the keys)."""
+    head 2^-18 of each other, V sizes that jump by powers of two between regions of two 64-key tiles
+    (at 500 keys in whole blocks: the exponent changes within one walk of the keys)."""
     from lagunalab_amd.q8_attn import q8_prefill_attention
     Hkv, cap = 2, n + 40
     assert _split(n, L, G, Hkv) == (n == 3000)
@@ -242,7 +242,7 @@ def test_prefill_operands_far_apart(dev, kind, n, L, G):
     elif kind == "V groups":
         v[..., 64:] *= np.float32(2.0 ** -18)
     else:
-        region = (np.arange(n) // 320) % 3
+        region = (np.arange(n) // 128) % 3
         k += np.where(region == 1, 6.0, -6.0).astype(np.float32)[:, None] * qdir[None, :, None, :]
         v *= (np.float32(2.0) ** np.array([4, -14, -5])[region]).astype(np.float32)[:, None]
     kq, vq = _buffers(dev, k, cap), _buffers(dev, v, cap)
