@@ -366,6 +366,26 @@ def q8_verify_append_attention(q, k_new, v_new, keys, values, n, scale):
     return out.to(q.dtype)
 
 
+def _two_verify_blocks_pay(B, Hkv, G, L, n):
+    """Whether a chunk of at most two verify blocks of P = min(16, 64 / G) positions is faster through
+    the verify kernel than as one half-filled block of the prefill kernel's exact-code form: long
+    contexts, where reading the cache twice is what the two launches cost. us, prefill kernel / verify
+    blocks: 17 rows, 24/8 heads, 16,000 keys 39 / 74, 65,000 94 / 83, 82,000 118 / 97; 48/8, 16,000
+    keys 45 / 80, 82,000 126 / 124, 8 sequences of 65,000 618 / 538, 32 of 4,000 165 / 196; with three
+    blocks (24 rows, 48/8, 82,000 keys) 152 / 170. Costs fitted to these: per block 12 us and, per
+    thousand cached rows of all KV heads, 0.044 to 0.069 by its query rows; the prefill kernel 25 us and
+    0.143; two launches from the host not under 76."""
+    P = min(16, 64 // G)
+    if G in (1, 2, 4, 8) or L > 2 * P:
+        return False
+    kkeys = B * Hkv * n / 1000
+    blocked = 0.06 * B * Hkv
+    for rows in (G * (L % P or P), G * P):
+        blocked += 12 + kkeys * (0.044 if rows <= 4 else 0.05 if rows <= 32 else 0.063 if rows <= 48
+                                 else 0.069)
+    return max(blocked, 76) < 25 + 0.143 * kkeys
+
+
 def q8_prefill_attention(q, keys, values, n, scale):
     """Causal attention of a prefill chunk over the 8-bit cache, without materializing the score
     matrix or a dequantized copy of the cache (the step before decode: ``L`` > 1 chunks on the
@@ -386,6 +406,8 @@ def q8_prefill_attention(q, keys, values, n, scale):
         return q8_verify_attention(q, keys, values, n, scale)
     if Hq // Hkv > 64:
         raise ValueError(f"{Hq // Hkv} query heads per KV head exceed 64")
+    if 16 < L <= 32 and _two_verify_blocks_pay(B, Hkv, Hq // Hkv, L, int(n)):
+        return _prefill_blocked(q, keys, values, n, scale)
     lib = _lib.load()
     vc, vs, vb = values
     dev = _lib.require_device(q, kc, ks, kb, vc, vs, vb)
@@ -418,8 +440,8 @@ def q8_prefill_attention(q, keys, values, n, scale):
 
 
 def _prefill_blocked(q, keys, values, n, scale):
-    """q8_prefill_attention's result from the verify kernel, a cross-check of the prefill kernel:
-    blocks of P = min(16, 64 / G) positions (one launch and one merge per block; a ragged first
+    """q8_prefill_attention from the verify kernel, for chunks of two blocks over long contexts (and a
+    cross-check of the prefill kernel): blocks of P = min(16, 64 / G) positions (one launch and one merge per block; a ragged first
     block of L mod P rows), each block over the keys its last row sees."""
     lib = _lib.load()
     B, Hq, L, D = q.shape

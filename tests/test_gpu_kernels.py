@@ -1069,3 +1069,26 @@ def test_dequantize_of_many_short_heads(dev, bits, gs, D, n, cap, B, H):
                 + b.float().repeat_interleave(gs, -1)).to(torch.bfloat16)
         assert torch.equal(got, want)
         assert torch.equal(dequantize(*buf, gs, bits, n=n), want)
+
+
+@pytest.mark.parametrize("L", [17, 20])
+def test_two_verify_blocks_equal_the_prefill_kernel(dev, L):
+    """17 and 20 rows at 48/8 heads over 8 sequences of 20,000 keys go through two verify blocks: the
+    function against the prefill kernel's entry."""
+    from lagunalab_amd import _lib, q8_attn
+    from lagunalab_amd.quant import quantize
+    lib = _lib.load()
+    n, G, Hkv, B = 20000, 6, 8, 8
+    assert q8_attn._two_verify_blocks_pay(B, Hkv, G, L, n)
+    g = torch.Generator(device=dev).manual_seed(L)
+    rnd = lambda *s: torch.randn(s, device=dev, generator=g).to(torch.bfloat16)  # noqa: E731
+    kq, vq = (quantize(rnd(B, Hkv, n, 128), 64, 8) for _ in range(2))
+    q = rnd(B, Hkv * G, L, 128)
+    got = q8_attn.q8_prefill_attention(q, kq, vq, n, 0.09)
+    need = lib.lq_prefill_workspace_bytes(B, Hkv * G, Hkv, L, n)
+    ws = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
+    out = torch.empty_like(q)
+    assert lib.lq_q8_prefill_attn_grouped(q.data_ptr(), *(t.data_ptr() for t in (*kq, *vq)), B, Hkv * G,
+                                          Hkv, L, 128, n, n, 0.09, out.data_ptr(), ws.data_ptr(), need,
+                                          _lib.stream_ptr(dev)) == _lib.LQ_OK
+    assert_attn_close(got, out.float().cpu().numpy(), "two verify blocks")
