@@ -36,8 +36,8 @@
 // P.V(t-1), so one fp16 K and one V^T buffer suffice. The codes of raw tile t+2 and the words of
 // t+3 go into t's slots once both dequantizations of t are done, from each half's softmax slot, and
 // are waited for a tile later. Vector phases run at a raised wave priority: their instructions set
-// the pace and the matrix phases' issue only every 16 cycles (2,048 rows at 82,671 keys: 2,437 ->
-// 2,407 us against 2,429 and 2,414 of an unchanged kernel beside them).
+// the pace and the matrix phases' issue only every 16 cycles (2,048 rows at 82,671 keys, in four turns
+// beside the kernel without it: 2,571-2,576 -> 2,549-2,551 us).
 // Tiles past a wave's last row are skipped by that wave (it keeps its copy and dequantization
 // duties); tiles straddling its rows' bounds are masked per row. Rows past the chunk (a ragged last
 // block) read no q and store nothing. Keys past n-1 are never read: copies clamp their rows to n-1.
@@ -56,7 +56,7 @@
 //  * A NaN or infinity in a key's words reaches the rows that see that key: no factor is taken from
 //    it, and masked tiles leave the terms of keys past a row's bound out.
 // That is 350 VALU instructions more per 32 rows and 128 keys, and twice the registers for P, so the
-// tiles are of 64 keys. Per 128 keys 7.1 us against 4.0 (clock 1.8-2.1 GHz), VALU-bound in the softmax
+// tiles are of 64 keys. Per 128 keys 7.0 us against 4.0 (clock 1.8-2.1 GHz), VALU-bound in the softmax
 // slots and about half of the Q.K^T slots: 512 rows at 8,193 keys, 48/8 heads, 190 us (in blocks of 10
 // positions through the verify kernel, each a launch that reads the whole cache and a merge, 1,010).
 // Without the raised wave priority 197, without the order of MFMAs and sums in qk() 196; the terms

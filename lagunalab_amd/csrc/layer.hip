@@ -514,8 +514,8 @@ typedef float facc_t __attribute__((ext_vector_type(4)));
 // (one 16x16x32 MFMA per 32 of it: A = 16 weight rows, B = the rows of x, rows past M repeating
 // the last), 8 steps' loads in flight; the waves' fp32 sums meet in LDS. Bound by the weights'
 // stream and its ramp (25 and 17 MB, 3-5 us at a large copy's rate) and by the rows of x that
-// every workgroup reads: 8 rows, 6,176 x 2,048 in 9.4 us and 2,048 x 4,096 in 8.1, where the
-// library takes 12.9 and 11.6 (in a graph, weights not cached).
+// every workgroup reads: 8 rows, 6,176 x 2,048 in 8.8 us and 2,048 x 4,096 in 8.3, where the
+// library takes 12.4 and 14.3 (in a graph, weights not cached).
 constexpr int GW = 8;
 __global__ __launch_bounds__(64 * GW) void gemm_rows_kernel(const uint16_t* __restrict__ W,
                                                             const uint16_t* __restrict__ x,
