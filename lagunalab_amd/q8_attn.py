@@ -376,7 +376,7 @@ def _two_verify_blocks_pay(B, Hkv, G, L, n):
     thousand cached rows of all KV heads, 0.044 to 0.069 by its query rows; the prefill kernel 25 us and
     0.143; two launches from the host not under 76."""
     P = min(16, 64 // G)
-    if G in (1, 2, 4, 8) or L > 2 * P:
+    if G in (1, 2, 4, 8) or L > 2 * P or B > 64 or B * Hkv > 2048:  # the verify kernel's limits
         return False
     kkeys = B * Hkv * n / 1000
     blocked = 0.06 * B * Hkv
