@@ -152,7 +152,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     ``lq_gemv_bf16`` (weight-streaming, HBM-bound), 2 to 16 rows (a verify block) the matrix-core
     form of it, ``lq_gemm_rows_bf16``, where it is faster, more rows the library GEMM."""
     K = x.shape[-1]
-    rows = x.numel() // K if K else 0
+    rows = x.numel() // K if K else 1  # no inputs: refused by the row's entry
     if rows != 1 and not (2 <= rows <= 16 and _row_form(x, w, rows, K)):
         return torch.matmul(x, w.t())
     lib = _lib.load()

@@ -121,3 +121,10 @@ def test_unwatched_calls_only_outside_tracing_modes_and_autocast():
 def test_row_form_only_where_it_was_measured_faster(rows, N, K, pays):
     from lagunalab_amd.attention import _row_form_pays
     assert _row_form_pays(rows, N, K) == bool(pays)
+
+
+def test_linear_refuses_rows_of_no_inputs():
+    import torch
+    from lagunalab_amd.attention import linear
+    with pytest.raises(ValueError):
+        linear(torch.empty((3, 0), dtype=torch.bfloat16), torch.empty((4, 0), dtype=torch.bfloat16))
