@@ -251,7 +251,7 @@ def quantized_scaled_dot_product_attention(queries, q_keys, q_values, scale, mas
     the first ``offset`` rows of the cache buffers; the kernel reads them in place (8- or 4-bit,
     group 64). Single query rows (the steps on which the cache exposes ``bits``) take the decode
     kernels; an 8-bit block of up to 16 rows with the bottom-right causal mask takes the verify
-    kernel. Returns ``[B, Hq, L, 128]`` in the queries' dtype."""
+    kernel (beyond 64 query rows per KV head the prefill kernel). Returns ``[B, Hq, L, 128]`` in the queries' dtype."""
     if group_size != 64:
         raise ValueError(f"quantized attention takes group_size 64, got {group_size}")
     B, Hq, L, D = queries.shape
@@ -271,7 +271,7 @@ def quantized_scaled_dot_product_attention(queries, q_keys, q_values, scale, mas
     if bits != 8 or L > 16 or mask not in ("causal",):
         raise ValueError("multi-row quantized attention takes the 8-bit cache, at most 16 rows "
                          "and the causal mask")
-    return q8_verify_attention(queries, keys, values, n, scale)
+    return q8_prefill_attention(queries, keys, values, n, scale)  # small blocks: the verify kernel
 
 
 def q8_verify_attention(q, keys, values, n, scale):

@@ -1014,7 +1014,7 @@ def test_blocks_of_more_than_64_query_rows_per_kv_head(dev, G, Hkv, L):
     prefill kernel (one row less than the limit, 60, through the verify kernel): the cache's protocol and
     the function against the oracle, the appended rows against a plain append."""
     from lagunalab_amd.cache import DequantKVCache, QuantizedKVCache
-    from lagunalab_amd.q8_attn import q8_prefill_attention
+    from lagunalab_amd.q8_attn import q8_prefill_attention, quantized_scaled_dot_product_attention
     rng = np.random.default_rng(G + L)
     n = 700
     k, v = (to_dev_bf16(Q.randn_bf16(rng, (1, Hkv, n + L, 128)), dev) for _ in range(2))
@@ -1031,6 +1031,9 @@ def test_blocks_of_more_than_64_query_rows_per_kv_head(dev, G, Hkv, L):
     assert_attn_close(out, want, "attend")
     assert_attn_close(q8_prefill_attention(to_dev_bf16(q, dev), plain.keys, plain.values, n + L, 0.09),
                       want, "function")
+    views = [tuple(t[:, :, :n + L] for t in x) for x in (plain.keys, plain.values)]
+    assert_attn_close(quantized_scaled_dot_product_attention(to_dev_bf16(q, dev), *views, 0.09,
+                                                             mask="causal"), want, "packed views")
 
 
 @pytest.mark.parametrize("L", [1, 3])
