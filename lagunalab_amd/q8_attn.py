@@ -366,24 +366,28 @@ def q8_verify_append_attention(q, k_new, v_new, keys, values, n, scale):
     return out.to(q.dtype)
 
 
-def _two_verify_blocks_pay(B, Hkv, G, L, n):
-    """Whether a chunk of at most two verify blocks of P = min(16, 64 / G) positions is faster through
-    the verify kernel than as one half-filled block of the prefill kernel's exact-code form: long
-    contexts, where reading the cache twice is what the two launches cost. us, prefill kernel / verify
-    blocks: 17 rows, 24/8 heads, 16,000 keys 39 / 74, 65,000 94 / 83, 82,000 118 / 97; 48/8, 16,000
-    keys 45 / 80, 82,000 126 / 124, 8 sequences of 65,000 618 / 538, 32 of 4,000 165 / 196; with three
-    blocks (24 rows, 48/8, 82,000 keys) 152 / 170. Costs fitted to these: per block 12 us and, per
-    thousand cached rows of all KV heads, 0.044 to 0.069 by its query rows; the prefill kernel 25 us and
-    0.143; two launches from the host not under 76."""
-    P = min(16, 64 // G)
-    if G in (1, 2, 4, 8) or L > 2 * P or B > 64 or B * Hkv > 2048:  # the verify kernel's limits
+def _verify_blocks_pay(B, Hkv, G, L, n):
+    """Whether a chunk is faster through the verify kernel, in blocks of P = min(16, 64 / G) positions,
+    than on the prefill kernel's exact-code form: where the query rows per KV head fill less than half of
+    a 256-row block (at most two verify blocks), or little of a second one, and the context is long, so
+    that reading the cache once per verify block is what those cost. us, prefill kernel / verify blocks:
+    17 rows, 24/8 heads, 16,000 keys 39 / 74, 65,000 94 / 83, 82,000 118 / 97; 48/8, 16,000 keys 45 / 80,
+    82,000 126 / 124, 8 sequences of 65,000 618 / 538, 32 of 4,000 165 / 196; three blocks (24 rows, 48/8,
+    82,000 keys) 152 / 170; 288 query rows (24 rows, 96/8, 32 sequences of 16,000 keys) 1,585 / 1,425, of
+    4,000 417 / 505. Costs fitted to these: per verify block 12 us, not under 38 from the host, and per
+    thousand cached rows of all KV heads 0.044 to 0.069 by its query rows; the prefill kernel 25 us and
+    0.143 (up to 128 rows) or 0.183 per 256-row block."""
+    P, R = min(16, 64 // G), G * L
+    if (G in (1, 2, 4, 8) or not (R <= 128 or 256 < R <= 320)
+            or B > 64 or B * Hkv > 2048):  # the verify kernel's limits
         return False
     kkeys = B * Hkv * n / 1000
-    blocked = 0.06 * B * Hkv
-    for rows in (G * (L % P or P), G * P):
-        blocked += 12 + kkeys * (0.044 if rows <= 4 else 0.05 if rows <= 32 else 0.063 if rows <= 48
-                                 else 0.069)
-    return max(blocked, 76) < 25 + 0.143 * kkeys
+    blocks = -(-L // P)
+    first = G * (L % P or P)  # query rows of the first, ragged block
+    cost = sum(0.044 if rows <= 4 else 0.05 if rows <= 32 else 0.063 if rows <= 48 else 0.069
+               for rows in (first,) + (G * P,) * (blocks - 1))
+    verify = max(12 * blocks + 0.06 * B * Hkv + kkeys * cost, 38 * blocks)
+    return verify < 25 + kkeys * (0.143 if R <= 128 else 0.183 * 2)
 
 
 def q8_prefill_attention(q, keys, values, n, scale):
@@ -406,7 +410,7 @@ def q8_prefill_attention(q, keys, values, n, scale):
         return q8_verify_attention(q, keys, values, n, scale)
     if Hq // Hkv > 64:
         raise ValueError(f"{Hq // Hkv} query heads per KV head exceed 64")
-    if 16 < L <= 32 and _two_verify_blocks_pay(B, Hkv, Hq // Hkv, L, int(n)):
+    if L > 16 and _verify_blocks_pay(B, Hkv, Hq // Hkv, L, int(n)):
         return _prefill_blocked(q, keys, values, n, scale)
     lib = _lib.load()
     vc, vs, vb = values
@@ -440,8 +444,8 @@ def q8_prefill_attention(q, keys, values, n, scale):
 
 
 def _prefill_blocked(q, keys, values, n, scale):
-    """q8_prefill_attention from the verify kernel, for chunks of two blocks over long contexts (and a
-    cross-check of the prefill kernel): blocks of P = min(16, 64 / G) positions (one launch and one merge per block; a ragged first
+    """q8_prefill_attention from the verify kernel, where _verify_blocks_pay says so (and a cross-check
+    of the prefill kernel): blocks of P = min(16, 64 / G) positions (one launch and one merge per block; a ragged first
     block of L mod P rows), each block over the keys its last row sees."""
     lib = _lib.load()
     B, Hq, L, D = q.shape

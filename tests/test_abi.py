@@ -225,7 +225,8 @@ def test_prefill_split_where_it_was_measured_faster(lib, Hq, Hkv, L, ctx, split)
 @pytest.mark.parametrize("B,Hkv,G,L,n,pays", [
     (1, 8, 3, 17, 16000, 0), (1, 8, 3, 17, 82000, 1), (1, 8, 3, 32, 82000, 1), (1, 8, 3, 33, 82000, 0),
     (1, 8, 4, 17, 82000, 0), (1, 8, 6, 17, 16000, 0), (8, 8, 6, 20, 65000, 1), (8, 8, 6, 21, 65000, 0),
-    (32, 8, 6, 17, 4000, 0), (1, 8, 64, 17, 82000, 0), (64, 8, 6, 17, 65000, 1), (65, 8, 6, 17, 65000, 0)])
-def test_two_verify_blocks_instead_of_a_half_filled_prefill_block(B, Hkv, G, L, n, pays):
-    from lagunalab_amd.q8_attn import _two_verify_blocks_pay
-    assert _two_verify_blocks_pay(B, Hkv, G, L, n) == bool(pays)
+    (32, 8, 6, 17, 4000, 0), (1, 8, 64, 17, 82000, 0), (64, 8, 6, 17, 65000, 1), (65, 8, 6, 17, 65000, 0), (32, 8, 12, 24, 16000, 1), (32, 8, 12, 24, 4000, 0),
+    (32, 8, 12, 27, 16000, 0), (1, 8, 6, 45, 82000, 0)])
+def test_verify_blocks_instead_of_part_filled_prefill_blocks(B, Hkv, G, L, n, pays):
+    from lagunalab_amd.q8_attn import _verify_blocks_pay
+    assert _verify_blocks_pay(B, Hkv, G, L, n) == bool(pays)

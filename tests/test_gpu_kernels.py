@@ -1074,15 +1074,15 @@ def test_dequantize_of_many_short_heads(dev, bits, gs, D, n, cap, B, H):
         assert torch.equal(dequantize(*buf, gs, bits, n=n), want)
 
 
-@pytest.mark.parametrize("L", [17, 20])
-def test_two_verify_blocks_equal_the_prefill_kernel(dev, L):
-    """17 and 20 rows at 48/8 heads over 8 sequences of 20,000 keys go through two verify blocks: the
-    function against the prefill kernel's entry."""
+@pytest.mark.parametrize("L", [17, 20, 43])
+def test_verify_blocks_equal_the_prefill_kernel(dev, L):
+    """17 and 20 rows (two verify blocks) and 43 (five) at 48/8 heads over 8 sequences of 20,000 keys go
+    through the verify kernel: the function against the prefill kernel's entry."""
     from lagunalab_amd import _lib, q8_attn
     from lagunalab_amd.quant import quantize
     lib = _lib.load()
     n, G, Hkv, B = 20000, 6, 8, 8
-    assert q8_attn._two_verify_blocks_pay(B, Hkv, G, L, n)
+    assert q8_attn._verify_blocks_pay(B, Hkv, G, L, n)
     g = torch.Generator(device=dev).manual_seed(L)
     rnd = lambda *s: torch.randn(s, device=dev, generator=g).to(torch.bfloat16)  # noqa: E731
     kq, vq = (quantize(rnd(B, Hkv, n, 128), 64, 8) for _ in range(2))
